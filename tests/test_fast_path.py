@@ -1,0 +1,134 @@
+"""The compiled code's common path (xt_fast.h) on the host against the
+oracle, bit for bit, at the edges of its forms and guards; the statements
+behind its exact quotients at small precisions."""
+import numpy as np
+import pytest
+
+import xtrack_amd as xt
+from fast_path_cases import CASES, IDS, edge_particles
+from helpers import compare_exact, random_particles
+from oracle_backend import GeneratedHostBackend, OracleBackend
+
+
+def _both(make, p, **kw):
+    out = []
+    for backend in (GeneratedHostBackend(), OracleBackend()):
+        line = make()
+        line.build_tracker(backend=backend)
+        q = p.copy()
+        line.track(q, **kw)
+        out.append(q)
+    return out
+
+
+@pytest.mark.parametrize('name,make,args', CASES, ids=IDS)
+def test_edges_of_forms_and_guards(name, make, args):
+    beam = random_particles(300, seed=2, scale=8e-4, p0c=7e12)
+    for p in (edge_particles(600, seed=1), beam):
+        a, b = _both(lambda: make(*args), p, num_turns=2)
+        assert not compare_exact(a, b)
+
+
+def test_structure_code_edges():
+    """The same elements among 70 records of their own strengths, which get
+    structure functions with loaded constants."""
+    def make():
+        els = []
+        for k in range(24):
+            els += [xt.Bend(length=3.0, angle=0.003 * (1 + 0.01 * k), knl=[0, 0, 1e-3 * k]),
+                    xt.Quadrupole(length=0.5, k1=0.1 * (-1) ** k * (1 + 0.02 * k)),
+                    xt.Multipole(knl=[0, 0.001 * k, 0.1]), xt.Drift(length=0.2 + 0.01 * k),
+                    xt.LimitRect(min_x=-0.02, max_x=0.02 + 1e-4 * k, min_y=-0.02, max_y=0.02)]
+        return xt.Line(elements=els)
+
+    for p in (edge_particles(500, seed=3), random_particles(300, seed=4, scale=1e-3, p0c=7e12)):
+        a, b = _both(make, p, num_turns=2)
+        assert not compare_exact(a, b)
+
+
+# -- arithmetic at p bits: integers m stand for m 2^e --------------------------
+def _rn(m, e, p):
+    """Round m 2^e to p bits, to nearest, ties to even."""
+    n = np.zeros_like(m)
+    t = np.abs(m)
+    for s in (32, 16, 8, 4, 2, 1):
+        big = (t >> s) > 0
+        n = n + np.where(big, s, 0)
+        t = np.where(big, t >> s, t)
+    k = np.maximum(n + 1 - p, 0)
+    a, half = np.abs(m), np.where(k > 0, 1 << np.maximum(k - 1, 0), 0)
+    q = a >> k
+    r = a - (q << k)
+    up = (k > 0) & ((r > half) | ((r == half) & (q & 1 == 1)))
+    return np.sign(m) * (q + up), e + k
+
+
+def _add(m1, e1, m2, e2):
+    e = np.minimum(e1, e2)
+    return (m1 << (e1 - e)) + (m2 << (e2 - e)), e
+
+
+def _div_rn(A, B, p):
+    """RN(A/B) for A, B of p bits: quotient with a sticky bit."""
+    q = (A << (p + 4)) // B
+    sticky = (q * B != (A << (p + 4))).astype(np.int64)
+    return _rn((q << 1) | sticky, np.full_like(q, -p - 5), p)
+
+
+@pytest.mark.parametrize('p', range(4, 12))
+def test_one_correction_rounds_every_quotient(p):
+    """q = RN(a y), r = a - q b, RN(q + r y) with y = RN(1/b) is RN(a/b), and
+    RN(y' + (1 - b y') y') is RN(1/b) from both neighbours y' of 1/b, from
+    the upper one also for b of all ones: every pair of p-bit significands."""
+    A, B = np.meshgrid(*[np.arange(1 << (p - 1), 1 << p, dtype=np.int64)] * 2, indexing='ij')
+    sc = np.full_like(A, -(p - 1))          # a = A 2^sc, b = B 2^sc
+    ym, ye = _div_rn(np.full_like(B, 1 << (p - 1)), B, p)
+    qm, qe = _rn(A * ym, sc + ye, p)
+    rm, re = _rn(*_add(A, sc, -qm * B, qe + sc), p)
+    q1 = _rn(*_add(qm, qe, rm * ym, re + ye), p)
+    want = _div_rn(A, B, p)
+    d, _ = _add(q1[0], q1[1], -want[0], want[1])
+    assert not d.any()
+    b = np.arange(1 << (p - 1), 1 << p, dtype=np.int64)
+    sc = np.full_like(b, -(p - 1))
+    one, zero = np.ones_like(b), np.zeros_like(b)
+    ym, ye = _div_rn(np.full_like(b, 1 << (p - 1)), b, p)
+    for k in (0, 1):
+        y1 = (1 << (2 * p - 1)) // b + k
+        e1 = np.full_like(b, -p)
+        if k:
+            y1 = np.where((1 << (2 * p - 1)) % b == 0, y1 - 1, y1)
+        rm, re = _rn(*_add(one, zero, -b * y1, sc + e1), p)
+        y2 = _rn(*_add(y1, e1, rm * y1, re + e1), p)
+        d, _ = _add(y2[0], y2[1], -ym, ye)
+        assert not (d if k else d[:-1]).any()
+
+
+@pytest.mark.parametrize('p', range(8, 13))
+def test_quotient_by_a_number_next_to_one(p):
+    """The polar drift's quotient t/den with d = 1 - den: q = RN(t + t w),
+    w = d + d^2 + d^3 (a power less than the code takes), corrected once with
+    y = RN(1 + w), for every t and every den with |d| < 2^-(p/3) but 1 - 2^-p."""
+    T = np.arange(1 << (p - 1), 1 << p, dtype=np.int64)
+    lim = 2.0 ** -((p + 2) // 3)
+    for side in (-1, 1):
+        e_d = -p if side < 0 else -(p - 1)
+        for k in range(2 if side < 0 else 1, 1 << p):
+            if k * 2.0 ** e_d >= lim:
+                break
+            full = lambda v: np.full_like(T, v)
+            dm, de = full(-side * k), full(e_d)
+            den = full((1 << -e_d) + side * k)
+            wm, we = _rn(*_add(dm, de, dm * dm, 2 * de), p)
+            wm, we = _rn(*_add(wm * dm, we + de, dm, de), p)
+            ym, ye = _rn(*_add(full(1), full(0), wm, we), p)
+            te = full(-(p - 1))
+            qm, qe = _rn(*_add(T, te, T * wm, te + we), p)
+            rm, re = _rn(*_add(T, te, -qm * den, qe + e_d), p)
+            q1 = _rn(*_add(qm, qe, rm * ym, re + ye), p)
+            B = (1 << p) - k if side < 0 else (1 << (p - 1)) + k
+            wantm, wante = _div_rn(T, full(B), p)
+            if side < 0:
+                wante = wante + 1          # den = B 2^-p, t = T 2^-(p-1)
+            d, _ = _add(q1[0], q1[1], -wantm, wante)
+            assert not d.any(), (side, k)

@@ -28,7 +28,7 @@ occupancy 3, 4 or 5 waves per SIMD for the interpreter kernel.  The
 compiled batch code is built for 5 waves per SIMD, so for a compiled batch
 only the block size is searched (``waves_per_eu`` sets the compiled code's
 occupancy target, 0 for the library default).  The per-thread LDS slots of the particle
-state are sized by the launch (block size x 48 bytes), so every block size
+state are sized by the launch (block size x 88 bytes), so every block size
 runs the same code.
 """
 import ctypes

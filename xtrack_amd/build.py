@@ -35,6 +35,7 @@ def _run(cmd):
 # headers the generated line code includes; embedded in the library so that
 # run-time compilation needs no source tree
 EMBEDDED_HEADERS = (('xt_math.h', CSRC), ('xt_program.h', CSRC), ('xt_ops.h', CSRC),
+                    ('xt_fast.h', CSRC),
                     ('xtrack_amd.h', os.path.join(ROOT, 'include')))
 _DELIM = 'XTMHDR'
 

@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
+#include <tuple>
 #include <string>
 #include <vector>
 
@@ -196,9 +197,416 @@ struct Gen {
     }
 };
 
-}  // namespace
 
-namespace {
+/* The unit code of one record or of a segment of records: the maps of
+   xt_fast.h in order, with the guards that their folded forms need.  The
+   generator follows bounds on |x|, |y|, |px| and |py| through the unit
+   (constants known; kInf where they are loaded) and whether px, py and zeta
+   can be -0, and writes a guard only where one is not already implied. */
+struct FastGen {
+    const std::vector<double> &prog;
+    const bool loads;
+    std::string out;
+    bool direct = false;   // holds an op that only the general code has
+    bool clear = false;    // ends with ax = ay = 0
+
+    FastGen(const std::vector<double> &p, bool l) : prog(p), loads(l) {}
+
+    static constexpr double kInf = 1e300;
+    static constexpr double kRange = 0x1p100;   // products of a few stay finite
+    static constexpr int kMaxDrifts = 64;
+    int64_t base = 0;
+    double bx = kInf, by = kInf, bpx = kInf, bpy = kInf;
+    bool signs = false;
+
+    std::string c(int64_t i) const {
+        if (loads) return "rp[" + std::to_string(i - base) + "]";
+        return lit(prog[i]);
+    }
+    std::string cs(int64_t i, int n) const {
+        std::string s;
+        for (int k = 0; k < n; k++) s += ", " + c(i + k);
+        return s;
+    }
+    void line(const std::string &s) { out += "    " + s + "\n"; }
+
+    void guard_range() {
+        if (bx <= kRange && by <= kRange && bpx <= kRange && bpy <= kRange) return;
+        line("xt::f_guard_range(p);");
+        bx = by = bpx = bpy = 1.0;
+    }
+    void guard_signs() {
+        if (!signs) line("xt::f_guard_signs(p);");
+        signs = true;
+    }
+
+    /* Checks of one convex limit (a LimitRect, the global limit) along
+       drifts: with px and py unchanged and lengths of one sign, x and y run
+       monotonically (rounding is monotone), so a check between two others of
+       the same limit is implied by them.  `held` is the place of the last
+       check, not written yet. */
+    struct Convex {
+        std::string text;      // the anchored check; empty: none
+        int64_t held = -1;     // place in out of the check held back
+        int sign = 0;          // sign of the drift lengths since the anchor
+    };
+    Convex rect, glob;
+
+    void flush(Convex &v, Convex &other) {
+        if (v.held >= 0) {
+            const std::string t = "    " + v.text + "\n";
+            out.insert((size_t)v.held, t);
+            if (other.held > v.held) other.held += (int64_t)t.size();
+        }
+        v = Convex();
+    }
+    void flush_limits() {
+        flush(rect, glob);
+        flush(glob, rect);
+    }
+    void drifted(double length) {
+        const int sg = length > 0 ? 1 : length < 0 ? -1 : 0;
+        for (Convex *v : {&rect, &glob}) {
+            if (v->text.empty()) continue;
+            if (loads || sg == 0 || (v->sign != 0 && v->sign != sg)) {
+                flush(*v, v == &rect ? glob : rect);
+            } else {
+                v->sign = sg;
+            }
+        }
+    }
+    void convex(Convex &v, const std::string &check) {
+        if (v.text == check) {
+            v.held = (int64_t)out.size();
+            return;
+        }
+        flush(v, &v == &rect ? glob : rect);
+        line(check);
+        v.text = check;
+    }
+
+    bool in_range(int64_t pos, int64_t n) const {
+        return pos >= 0 && n >= 0 && pos + n <= (int64_t)prog.size();
+    }
+
+    struct Polar { int64_t length, consts; };   // program indices: length; ca sa t2 ica
+
+    /* Bounds through a chain of polar drifts of curvature radius rho with
+       kicks px -= kick[j] after drift j, from |x| <= 1, |px| <= p0, |py| <=
+       1/4, |delta| <= 1/4: 0 when they leave the ranges of f_polar, 2 when
+       its small-angle form holds, else 1; the bounds on x and px at the end. */
+    int polar_plan(const std::vector<Polar> &d, const std::vector<double> &kick, double rho,
+                   double p0, double *x_end, double *px_end) const {
+        double xb = 1.0, lo = -p0, hi = p0;
+        bool small = true;
+        for (size_t j = 0; j < d.size(); j++) {
+            const double ca = prog[d[j].consts], sa = prog[d[j].consts + 1];
+            const double t2 = prog[d[j].consts + 2], ica = prog[d[j].consts + 3];
+            if (ica == 0.0) return 0;
+            const double pm = std::max(-lo, hi);
+            if (!(pm <= 0.25)) return 0;
+            const double pz_lo = std::sqrt(0.5625 - 0.0625 - pm * pm), pz_hi = 1.25;
+            const double w = std::fabs(sa) * pm / pz_lo;
+            if (!(w / ca <= 0x1.6p-15)) small = false;   // below 2^-14.5
+            xb = (xb + std::fabs(rho) * (t2 + w)) / (ca - w);
+            if (!(xb <= 0x1p20) || !(std::fabs(rho) >= 2 * xb)) return 0;
+            const double s_lo = std::min(sa * pz_lo, sa * pz_hi);
+            const double s_hi = std::max(sa * pz_lo, sa * pz_hi);
+            lo = (lo < 0 ? lo : ca * lo) + s_lo;
+            hi = (hi > 0 ? hi : ca * hi) + s_hi;
+            if (j < kick.size()) {
+                lo -= kick[j];
+                hi -= kick[j];
+            }
+            lo -= 0x1p-40;
+            hi += 0x1p-40;
+        }
+        if (!(std::max(-lo, hi) <= 0.25)) return 0;
+        *x_end = xb;
+        *px_end = std::max(-lo, hi);
+        return small ? 2 : 1;
+    }
+
+    /* drifts d with kicks (program index of the strength, times the word at
+       L) between them */
+    void polar_chain(int64_t rho, const std::vector<Polar> &d, const std::vector<int64_t> &kick,
+                     int64_t L) {
+        std::vector<double> kv;
+        for (int64_t k : kick) kv.push_back(prog[k] * prog[L]);
+        double xe = 0, pe = 0, p0 = 0x1p-7;
+        int plan = polar_plan(d, kv, prog[rho], p0, &xe, &pe);
+        if (plan != 2) {
+            p0 = 0x1p-4;
+            plan = polar_plan(d, kv, prog[rho], p0, &xe, &pe);
+        }
+        if (plan == 0) {
+            direct = true;
+            return;
+        }
+        line("xt::f_polar_guard(p, " + lit(p0) + ");");
+        for (size_t j = 0; j < d.size(); j++) {
+            line(std::string("xt::f_polar<") + (plan == 2 ? "true" : "false") + ">(p, " +
+                 c(d[j].length) + ", " + c(rho) + cs(d[j].consts, 4) + ");");
+            if (j < kick.size()) line("p.px = p.px - " + c(kick[j]) + " * " + c(L) + ";");
+        }
+        double ell = 0;
+        for (auto &v : d) ell += std::fabs(prog[v.length]);
+        bx = xe;
+        bpx = pe;
+        bpy = 0.25;
+        by += 4 * ell;
+    }
+
+    /* one folded Horner pass (xt_ops.h: horner_step, kick_pass_apply); a sum
+       that is known to be zero is left out */
+    bool kick_pass(int64_t fp, const std::string &w, double wv, double *dpx_b, double *dpy_b) {
+        if (!in_range(fp, 1)) return false;
+        const int64_t top = wbits(prog[fp]);
+        if (top < -1 || top > 1000 || !in_range(fp, 2 * top + 3)) return false;
+        if (top < 0) return true;
+        const int64_t ia = fp + 1, ib = fp + 2 + top;
+        bool zx = prog[ia + top] == 0.0, zy = prog[ib + top] == 0.0;
+        line("{");
+        line("    double dpx = " + (zx ? std::string("0.0") : c(ia + top)) + ", dpy = " +
+             (zy ? std::string("0.0") : c(ib + top)) + ", zre, zim;");
+        double b = std::fabs(prog[ia + top]) + std::fabs(prog[ib + top]);
+        for (int64_t k = top - 1; k >= 0; k--) {
+            if (zx && zy) return false;   // top is the highest non-zero coefficient
+            line(std::string("    zre = ") + (zx ? "-(dpy * y)" : zy ? "dpx * x"
+                                                                     : "dpx * x - dpy * y") + ";");
+            line(std::string("    zim = ") + (zx ? "dpy * x" : zy ? "dpx * y"
+                                                                  : "dpx * y + dpy * x") + ";");
+            zx = zy = false;
+            line("    dpx = " + (prog[ia + k] != 0.0 ? c(ia + k) + " + zre" : "zre") + ";");
+            line("    dpy = " + (prog[ib + k] != 0.0 ? c(ib + k) + " + zim" : "zim") + ";");
+            b = b * (bx + by) + std::fabs(prog[ia + k]) + std::fabs(prog[ib + k]);
+        }
+        if (!zx) line("    p.px = p.px + " + w + " * (-dpx);");
+        if (!zy) line("    p.py = p.py + " + w + " * dpy;");
+        line("}");
+        *dpx_b += std::fabs(wv) * b;
+        *dpy_b += std::fabs(wv) * b;
+        return true;
+    }
+
+    bool kick(int64_t pc) {
+        const double *a = &prog[pc + 1];
+        const std::string w = c(pc + 1);
+        const int64_t desc = wbits(a[1]), mask = wbits(a[2]);
+        if (!in_range(desc, KD_ARR)) return false;
+        guard_range();
+        guard_signs();
+        double dx = 0, dy = 0;
+        line("{");
+        line("const double x = p.x, y = p.y;");
+        line("(void)x; (void)y;");
+        for (int k = 0; k < 3; k++)
+            if ((mask & (1 << k)) &&
+                !kick_pass(wbits(prog[desc + KD_FASTOFF + k]), w, a[0], &dx, &dy))
+                return false;
+        if (mask & (8 | 16 | 32))
+            line(std::string("xt::f_curvature(p, x, y, ") + ((mask & 8) ? "true" : "false") +
+                 ", " + ((mask & 16) ? "true" : "false") + ", " + ((mask & 32) ? "true" : "false") +
+                 cs(pc + 4, 3) + ");");
+        line("}");
+        dx += 2 * std::fabs(a[3]) + std::fabs(a[4]) * bx + std::fabs(a[5]) * (bx * bx + by * by);
+        dy += std::fabs(a[5]) * bx * by;
+        // the same code serves records with other strengths
+        bpx = loads ? kInf : bpx + dx;
+        bpy = loads ? kInf : bpy + dy;
+        return true;
+    }
+
+    void quad(int64_t a) {
+        const double L = prog[a], k0 = prog[a + 1], k1 = prog[a + 2], h = prog[a + 3];
+        const double k = std::fabs(k1), ph = 4.0 / 3.0 * k * L * L;
+        // phase sqrt(k1 / (1 + delta)) L in [2^-20, pi/4], |delta| <= 1/4
+        if (wbits(k0) != 0 || wbits(h) != 0 || !(k >= 0x1p-20 && k <= 0x1p20) ||
+            !(0.8 * k * L * L >= 0x1p-40) || !(ph <= 0.61) || !(std::fabs(L) <= 0x1p20)) {
+            direct = true;
+            return;
+        }
+        guard_range();
+        guard_signs();
+        line(std::string("xt::f_quad<") + (k1 > 0 ? "true" : "false") + ">(p, " + c(a) + ", " +
+             c(a + 2) + ");");
+        const double x = 2 * bx + 4 * std::fabs(L) * bpx, y = 2 * by + 4 * std::fabs(L) * bpy;
+        bpx = 4 * bpx + 4 * k * std::fabs(L) * bx;
+        bpy = 4 * bpy + 4 * k * std::fabs(L) * by;
+        bx = x;
+        by = y;
+        if (loads) bx = by = bpx = bpy = kInf;
+    }
+
+    static int drifts(int64_t op) {
+        return op == OP_YOSHIDA4_BEND ? 4 : op == OP_YOSHIDA6_BEND ? 8 : op == OP_POLAR ? 1 : 0;
+    }
+
+    bool same_op(int64_t p, int64_t q) const {
+        const int64_t op = wbits(prog[p]);
+        return op == wbits(prog[q]) &&
+               std::memcmp(&prog[p + 1], &prog[q + 1], sizeof(double) * kNargs[op]) == 0;
+    }
+
+    /* append record pc; false for a program this generator cannot read.  A
+       strong bend is integrated in hundreds of equal steps: the largest
+       repetition of its ops becomes a loop, and a bend that still holds more
+       than kMaxDrifts polar drifts is left to the general code (straight-line
+       code for 576 drifts compiles in minutes). */
+    bool record(int64_t pc) {
+        base = pc;
+        std::vector<int64_t> ops;
+        int n_drifts = 0;
+        for (;;) {
+            if (!in_range(pc, 1) || ops.size() > 100000) return false;
+            const int64_t op = wbits(prog[pc]);
+            if (op < 0 || op >= OP_NUM) return false;
+            if (op == OP_END) break;
+            if (!in_range(pc + 1, kNargs[op])) return false;
+            ops.push_back(pc);
+            n_drifts += drifts(op);
+            pc += 1 + kNargs[op];
+        }
+        // ops [first, first + period * count) repeat the first period
+        size_t first = 0, period = 0, count = 0;
+        if (n_drifts > kMaxDrifts) {
+            for (size_t f = 0; f < ops.size() && f < 8; f++)
+                for (size_t q = 1; 2 * q <= ops.size() - f && q <= 64; q++) {
+                    size_t e = f + q;
+                    while (e < ops.size() && same_op(ops[e], ops[e - q])) e++;
+                    const size_t r = (e - f) / q;
+                    if (r > 1 && (r - 1) * q > (count ? (count - 1) * period : 0)) {
+                        first = f;
+                        period = q;
+                        count = r;
+                    }
+                }
+            for (size_t k = first; count && k < first + period * (count - 1); k++)
+                n_drifts -= drifts(wbits(prog[ops[k]]));
+            if (n_drifts > kMaxDrifts) {
+                direct = true;
+                return true;
+            }
+        }
+        axay = false;
+        for (size_t k = 0; k < ops.size(); k++) {
+            if (count && k == first) {
+                flush_limits();
+                bx = by = bpx = bpy = kInf;   // as every repetition finds them
+                signs = false;
+                out += "#pragma clang loop unroll(disable)\n";
+                line("for (int step = 0; step < " + std::to_string(count) + "; step++) {");
+            }
+            if (!emit(ops[k])) return false;
+            if (direct) return true;
+            if (count && k == first + period - 1) {
+                flush_limits();
+                line("}");
+                k = first + period * count - 1;
+            }
+        }
+        // an entry edge without its exit leaves its own ax, ay
+        if (axay) direct = true;
+        return true;
+    }
+
+    bool axay = false;
+
+    bool emit(int64_t pc) {
+        const int64_t op = wbits(prog[pc]);
+        const int64_t a = pc + 1;
+        if (op != OP_DRIFT_EXP && op != OP_LIMIT_RECT && op != OP_LIMIT_ELLIPSE &&
+            op != OP_GLOBAL_APER)
+            flush_limits();
+        switch (op) {
+        case OP_DRIFT_EXP: {
+            drifted(prog[a]);
+            line("xt::f_drift(p, " + c(a) + ");");
+            const double l = loads ? kInf : 8 * std::fabs(prog[a]);
+            bx += l * bpx;
+            by += l * bpy;
+            break; }
+        case OP_DRIFT_EXACT: {
+            line("xt::f_drift_exact(p, " + c(a) + ");");
+            const double l = loads ? kInf : 2 * std::fabs(prog[a]);
+            bpx = bpy = 0.25;
+            bx += l;
+            by += l;
+            break; }
+        case OP_POLAR:
+            polar_chain(a + 1, {{a, a + 2}}, {}, a);
+            break;
+        case OP_YOSHIDA4_BEND:
+            polar_chain(a + 1, {{a + 4, a + 5}, {a + 9, a + 10}, {a + 9, a + 10},
+                                {a + 4, a + 5}}, {a + 2, a + 3, a + 2}, a);
+            break;
+        case OP_YOSHIDA6_BEND: {
+            std::vector<Polar> d;
+            std::vector<int64_t> k;
+            for (int j = 0; j < 8; j++) {
+                const int64_t q = a + 6 + 5 * (j < 4 ? j : 7 - j);
+                d.push_back({q, q + 1});
+                if (j < 7) k.push_back(a + 2 + (j < 4 ? j : 6 - j));
+            }
+            polar_chain(a + 1, d, k, a);
+            break; }
+        case OP_DIPQUAD: quad(a); break;
+        case OP_KICK:
+            if (!kick(pc)) return false;
+            break;
+        case OP_EDGE_AXAY: axay = true; break;
+        case OP_EDGE_CLEAR_AXAY:
+            axay = false;
+            clear = true;
+            break;
+        case OP_EDGE_LINEAR:
+            if (!loads && prog[a] == 0.0 && prog[a + 1] == 0.0) {
+                guard_range();
+                guard_signs();
+                break;
+            }
+            line("xt::f_edge_linear(p" + cs(a, 2) + ");");
+            bpx = loads ? kInf : bpx + std::fabs(prog[a]) * bx;
+            bpy = loads ? kInf : bpy + std::fabs(prog[a + 1]) * by;
+            break;
+        case OP_XY_SHIFT:
+            line("xt::f_xy_shift(p" + cs(a, 2) + ");");
+            bx += loads ? kInf : std::fabs(prog[a]);
+            by += loads ? kInf : std::fabs(prog[a + 1]);
+            break;
+        case OP_S_ROT: {
+            line("xt::f_s_rot(p" + cs(a, 2) + ");");
+            signs = false;
+            bx = by = 2 * (bx + by);
+            bpx = bpy = 2 * (bpx + bpy);
+            break; }
+        case OP_LIMIT_RECT:
+            if (!loads && prog[a] == -prog[a + 1] && prog[a + 2] == -prog[a + 3])
+                convex(rect, "xt::f_limit_rect_sym(p, " + c(a + 1) + ", " + c(a + 3) + ");");
+            else if (!loads)
+                convex(rect, "xt::f_limit_rect(p" + cs(a, 4) + ");");
+            else
+                line("xt::f_limit_rect(p" + cs(a, 4) + ");");
+            break;
+        case OP_LIMIT_ELLIPSE:
+            line("xt::f_limit_ellipse(p" + cs(a, 3) + ");");
+            break;
+        case OP_GLOBAL_APER: convex(glob, "xt::f_global_aper(p);"); break;
+        default:
+            // RF, frame rotations, exact bends: the general code
+            direct = true;
+            break;
+        }
+        return true;
+    }
+
+    std::string body() {
+        flush_limits();
+        if (direct) return "    p.bad = true;\n";
+        if (clear) line("p.clear = true;");
+        return out;
+    }
+};
 
 /* Functions of the generated code for a set of lines (one line, or the
    lines of a batch).  A record whose literal code serves at least two
@@ -211,10 +619,12 @@ namespace {
    records would be megabytes of instructions, streamed through the
    instruction cache once per turn. */
 struct CodeSet {
-    std::vector<std::string> body;             // function bodies
+    std::vector<std::string> body;             // function bodies (general code)
+    std::vector<std::string> fast;             // their unit code
     std::vector<char> small;                   // cheap literal records
     bool keyed_pc = false;                     // keys carry the program offset
     std::vector<std::vector<int32_t>> segs;    // segment function bodies
+    std::vector<std::string> fast_segs;        // their unit code
 };
 
 int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
@@ -235,13 +645,15 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     std::map<std::string, int64_t> lit_uses;
     std::vector<std::map<int64_t, std::string>> lit_text(nl);
     std::map<std::string, std::pair<bool, int>> lit_info;   // heavy, cost
-    std::map<std::string, std::string> struct_of_lit;
+    std::map<std::string, std::string> fast_of_lit, struct_of_lit;
     std::map<std::string, int64_t> lits_of_struct;         // distinct literal texts
     for (size_t l = 0; l < nl; l++)
         for (auto &pu : uses[l]) {
             Gen g(*progs[l], pu.first, false, !all_literal);
             Gen gs(*progs[l], pu.first, true);
-            if (!g.record(pu.first) || !gs.record(pu.first)) {
+            FastGen f(*progs[l], false), fs(*progs[l], true);
+            if (!g.record(pu.first) || !gs.record(pu.first) || !f.record(pu.first) ||
+                !fs.record(pu.first)) {
                 err = "cannot generate code for line " + std::to_string(l) +
                       " at program offset " + std::to_string(pu.first);
                 return XTM_ERR_ARG;
@@ -249,7 +661,12 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
             lit_uses[g.out] += pu.second;
             lit_info[g.out] = {g.heavy, g.cost};
             lit_text[l][pu.first] = g.out;
-            if (struct_of_lit.emplace(g.out, gs.out).second) lits_of_struct[gs.out]++;
+            fast_of_lit.emplace(g.out, f.body());
+            // a structure is its general and its unit code: records of one
+            // op sequence differ in the latter where a form depends on the
+            // ranges of their constants
+            const std::string st = gs.out + fs.body();
+            if (struct_of_lit.emplace(g.out, st).second) lits_of_struct[st]++;
         }
     // A structure that the set holds with many different constants (the
     // bends of ring variants with different cell counts) gets one structure
@@ -266,6 +683,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     for (auto &r : ranked) {
         fn_of_lit.emplace(*r.second, (int32_t)cs.body.size());
         cs.body.push_back(*r.second);
+        cs.fast.push_back(fast_of_lit[*r.second]);
         const auto &info = lit_info[*r.second];
         cs.small.push_back(!info.first && info.second <= kSmallCost);
     }
@@ -281,14 +699,17 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                 continue;
             }
             Gen g(*progs[l], pu.first, true);
-            if (!g.record(pu.first)) {
+            FastGen f(*progs[l], true);
+            if (!g.record(pu.first) || !f.record(pu.first)) {
                 err = "cannot generate code for line " + std::to_string(l) +
                       " at program offset " + std::to_string(pu.first);
                 return XTM_ERR_ARG;
             }
-            auto ins = fn_of_struct.emplace(g.out, (int32_t)cs.body.size());
+            const std::string fast = f.body();
+            auto ins = fn_of_struct.emplace(g.out + fast, (int32_t)cs.body.size());
             if (ins.second) {
                 cs.body.push_back(g.out);
+                cs.fast.push_back(fast);
                 cs.small.push_back(0);
             }
             fn_of_pc.emplace(pu.first, ins.first->second);
@@ -329,28 +750,45 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
             e = f;
         }
     }
-    auto chunk_seq = [&](const std::tuple<size_t, size_t, size_t> &ch) {
+    using Chunk = std::tuple<size_t, size_t, size_t>;
+    auto chunk_seq = [&](const Chunk &ch) {
         const std::vector<int32_t> &rv = recs[std::get<0>(ch)];
         return std::vector<int32_t>(rv.begin() + std::get<1>(ch),
                                     rv.begin() + std::get<1>(ch) + std::get<2>(ch));
     };
     std::map<std::vector<int32_t>, int64_t> count;
-    for (auto &ch : chunks) count[chunk_seq(ch)]++;
-    std::vector<std::pair<int64_t, const std::vector<int32_t> *>> seg_rank;
+    std::map<std::vector<int32_t>, Chunk> where;
+    for (auto &ch : chunks) {
+        count[chunk_seq(ch)]++;
+        where.emplace(chunk_seq(ch), ch);
+    }
+    std::vector<std::pair<int64_t, std::vector<int32_t>>> ranked_segs, seg_rank;
     for (auto &kv : count)
         if (kv.second >= 2)
-            seg_rank.emplace_back(kv.second * (int64_t)(kv.first.size() - 1), &kv.first);
-    std::stable_sort(seg_rank.begin(), seg_rank.end(),
+            ranked_segs.emplace_back(kv.second * (int64_t)(kv.first.size() - 1), kv.first);
+    std::stable_sort(ranked_segs.begin(), ranked_segs.end(),
                      [](const auto &x, const auto &y) { return x.first > y.first; });
-    std::map<std::vector<int32_t>, int32_t> seg_id;
     int64_t seg_body = 0;
-    for (auto &r : seg_rank) {
-        if ((int64_t)cs.segs.size() >= kSegMaxCount ||
-            seg_body + (int64_t)r.second->size() > kSegMaxBody)
+    for (auto &r : ranked_segs) {
+        if ((int64_t)seg_rank.size() >= kSegMaxCount ||
+            seg_body + (int64_t)r.second.size() > kSegMaxBody)
             continue;
-        seg_id.emplace(*r.second, (int32_t)cs.segs.size());
-        cs.segs.push_back(*r.second);
-        seg_body += (int64_t)r.second->size();
+        seg_body += (int64_t)r.second.size();
+        seg_rank.push_back(r);
+    }
+    std::map<std::vector<int32_t>, int32_t> seg_id;
+    for (auto &r : seg_rank) {
+        seg_id.emplace(r.second, (int32_t)cs.segs.size());
+        cs.segs.push_back(r.second);
+        const Chunk &ch = where[r.second];
+        FastGen f(*progs[std::get<0>(ch)], false);
+        for (size_t j = 0; j < std::get<2>(ch); j++)
+            if (!f.record((*entries[std::get<0>(ch)])[std::get<1>(ch) + j])) {
+                err = "cannot generate code for a segment of line " +
+                      std::to_string(std::get<0>(ch));
+                return XTM_ERR_ARG;
+            }
+        cs.fast_segs.push_back(f.body());
     }
     for (auto &ch : chunks) {
         auto it = seg_id.find(chunk_seq(ch));
@@ -368,7 +806,7 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
     s += std::string("// generated ") + what + ": element records as straight-line calls\n";
     if (options & XTM_SPEC_FAST_ARITH) s += "#define XTM_ARITH_FAST 1\n";
     s += "#if defined(__HIPCC__) && !defined(__HIPCC_RTC__)\n#include <hip/hip_runtime.h>\n#endif\n";
-    s += "#include \"xt_ops.h\"\n\n";
+    s += "#include \"xt_fast.h\"\n\n";
     s += "#if defined(__HIPCC__)\n#define XT_GEN_FN static __host__ __device__ __forceinline__\n";
     s += "#else\n#define XT_GEN_FN static inline\n#endif\n\n";
     s += "namespace xt_gen {\n";
@@ -380,6 +818,12 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
         s += cs.body[r];
         s += "}\n\n";
     }
+    for (size_t r = 0; r < cs.fast.size(); r++)
+        s += "XT_GEN_FN void fast_" + std::to_string(r) +
+             "(xt::FState &p, xt::CProg rp) {\n    (void)p; (void)rp;\n" + cs.fast[r] + "}\n\n";
+    for (size_t q = 0; q < cs.fast_segs.size(); q++)
+        s += "XT_GEN_FN void fast_seg_" + std::to_string(q) + "(xt::FState &p) {\n    (void)p;\n" +
+             cs.fast_segs[q] + "}\n\n";
     // a segment's records that address the program (relative literal code
     // of thin kicks: the literal kick's descriptor) get their own element's
     // rp from ent, the entry offsets from the chunk's first element on
@@ -417,8 +861,7 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
     const std::string rp = cs.keyed_pc
                                ? "        const xt::CProg rp = xt::cptr(prog) + xt::uniform(k.pc);\n"
                                : "        const xt::CProg rp = xt::cptr(prog);\n";
-    s += "    static constexpr bool kSegments = true;\n"
-         "    XT_HD static int32_t span(Key k) { return (" + kr + " >> " +
+    s += "    XT_HD static int32_t span(Key k) { return (" + kr + " >> " +
          std::to_string(XT_KEY_SPAN_SHIFT) + ") & " + std::to_string(XT_KEY_SPAN_MASK) +
          "; }\n"
          "    XT_HD int32_t segment(xt::PState<double> &p, const xt::PRef &m, Key k,\n"
@@ -438,6 +881,23 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
         s += "        case " + std::to_string(r) + ": rec_" + std::to_string(r) +
              "(p, m, prog, rp, c); break;\n";
     s += "        default: p.state = -999; break;\n"
+         "        }\n"
+         "    }\n"
+         "    /* the units of xt_fast.h */\n"
+         "    XT_HD void fast_segment(xt::FState &p, Key k) const {\n"
+         "        switch (" + kr + " >> " + std::to_string(XT_KEY_SEG_SHIFT) + ") {\n";
+    for (size_t q = 0; q < cs.segs.size(); q++)
+        s += "        case " + std::to_string(q + 1) + ": fast_seg_" + std::to_string(q) +
+             "(p); break;\n";
+    s += "        default: p.bad = true; break;\n"
+         "        }\n"
+         "    }\n"
+         "    XT_HD void fast(xt::FState &p, Key k) const {\n" + rp +
+         "        switch (" + kr + " & " + std::to_string(XT_KEY_REC_MASK) + ") {\n";
+    for (size_t r = 0; r < cs.body.size(); r++)
+        s += "        case " + std::to_string(r) + ": fast_" + std::to_string(r) +
+             "(p, rp); break;\n";
+    s += "        default: p.bad = true; break;\n"
          "        }\n"
          "    }\n"
          "};\n";
@@ -469,12 +929,13 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
          "    const xtm_monitor *__restrict__ Md, const xtm_particles *__restrict__ Pd,\n"
          "    uint64_t flags) {\n"
          "    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;\n"
-         "    if (i >= P.capacity) return;\n"
          "    const xt::TrackCtx c{flags, line_length, P.q0, P.t_sim};\n"
          "    // chi == 1 particles; the interpreter kernel tracks the others\n"
-         "    xt::track_particle_chi1(P, i, xt_gen::Runner{rec, entry, prog}, c, num_turns,\n"
-         "                            ele_start, num_ele_track, flag_end_turn_actions,\n"
-         "                            flag_reset_s, flag_monitor, xt::MonRef{Md, Pd});\n"
+         "    const bool alive = i < P.capacity && P.state[i] > 0 && P.chi[i] == 1.0;\n"
+         "    xt::track_particle_units(P, i, alive, xt_gen::Runner{rec, entry, prog}, c,\n"
+         "                             num_turns, ele_start, num_ele_track,\n"
+         "                             flag_end_turn_actions, flag_reset_s, flag_monitor,\n"
+         "                             xt::MonRef{Md, Pd});\n"
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over all particles\n"
@@ -485,11 +946,19 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
          "    xtm_monitor m0 = {};\n"
          "    const xt::TrackCtx c{flags, line_length, P->q0, P->t_sim};\n"
          "    const xt::MonRef mon{M ? M : &m0, P};\n"
-         "    for (int64_t i = 0; i < P->capacity; i++)\n"
-         "        xt::track_particle_with<false>(*P, i, xt_gen::Runner{rec, entry, prog},\n"
-         "                                xt::ProgramRunner{entry, prog}, c, num_turns,\n"
-         "                                ele_start, num_ele_track, flag_end_turn_actions,\n"
-         "                                flag_reset_s, flag_monitor, mon);\n"
+         "    for (int64_t i = 0; i < P->capacity; i++) {\n"
+         "        if (!(P->state[i] > 0)) continue;\n"
+         "        if (P->chi[i] == 1.0)\n"
+         "            xt::track_particle_units(*P, i, true, xt_gen::Runner{rec, entry, prog}, c,\n"
+         "                                     num_turns, ele_start, num_ele_track,\n"
+         "                                     flag_end_turn_actions, flag_reset_s,\n"
+         "                                     flag_monitor, mon);\n"
+         "        else\n"
+         "            xt::track_particle_loop_cold<false>(*P, i, xt::ProgramRunner{entry, prog},\n"
+         "                                     c, num_turns, ele_start, num_ele_track,\n"
+         "                                     flag_end_turn_actions, flag_reset_s,\n"
+         "                                     flag_monitor, mon);\n"
+         "    }\n"
          "}\n"
          "#endif\n";
     src = std::move(s);
@@ -521,16 +990,17 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "    const double *__restrict__ lengths, const xtm_particles *__restrict__ Pd,\n"
          "    int32_t num_turns, uint64_t flags) {\n"
          "    const xt_gen::BatchBlock b = xt::cptr(blocks)[blockIdx.x];\n"
-         "    if ((int32_t)threadIdx.x >= b.count) return;\n"
          "    const xtm_particles &P = *Pd;\n"
          "    const int64_t i = b.first + threadIdx.x;\n"
          "    const int64_t ne = xt::cptr(nele)[b.line];\n"
          "    const xt::TrackCtx c{flags, xt::cptr(lengths)[b.line], P.q0, P.t_sim, ne};\n"
          "    // chi == 1 particles; the interpreter batch kernel tracks the others\n"
-         "    xt::track_particle_chi1(P, i, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
-         "                            xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
-         "                            num_turns, 0, (int32_t)ne, 1, 1, 0,\n"
-         "                            xt::MonRef{nullptr, Pd});\n"
+         "    const bool alive = (int32_t)threadIdx.x < b.count && P.state[i] > 0 &&\n"
+         "                       P.chi[i] == 1.0;\n"
+         "    xt::track_particle_units(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
+         "                             xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
+         "                             num_turns, 0, (int32_t)ne, 1, 1, 0,\n"
+         "                             xt::MonRef{nullptr, Pd});\n"
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over the blocks\n"
@@ -542,11 +1012,18 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "        const xt_gen::BatchBlock b = blocks[bi];\n"
          "        const int64_t ne = nele[b.line];\n"
          "        const xt::TrackCtx c{flags, lengths[b.line], P->q0, P->t_sim, ne};\n"
-         "        for (int32_t t = 0; t < b.count; t++)\n"
-         "            xt::track_particle_with<false>(*P, b.first + t,\n"
-         "                xt_gen::Runner{recs[b.line], entries[b.line], progs[b.line]},\n"
-         "                xt::ProgramRunner{entries[b.line], progs[b.line]}, c, num_turns, 0,\n"
-         "                (int32_t)ne, 1, 1, 0, xt::MonRef{nullptr, P});\n"
+         "        const xt::MonRef mon{nullptr, P};\n"
+         "        for (int64_t i = b.first; i < b.first + b.count; i++) {\n"
+         "            if (!(P->state[i] > 0)) continue;\n"
+         "            if (P->chi[i] == 1.0)\n"
+         "                xt::track_particle_units(*P, i, true,\n"
+         "                    xt_gen::Runner{recs[b.line], entries[b.line], progs[b.line]}, c,\n"
+         "                    num_turns, 0, (int32_t)ne, 1, 1, 0, mon);\n"
+         "            else\n"
+         "                xt::track_particle_loop_cold<false>(*P, i,\n"
+         "                    xt::ProgramRunner{entries[b.line], progs[b.line]}, c, num_turns, 0,\n"
+         "                    (int32_t)ne, 1, 1, 0, mon);\n"
+         "        }\n"
          "    }\n"
          "}\n"
          "#endif\n";

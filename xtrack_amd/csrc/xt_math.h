@@ -220,8 +220,7 @@ XT_MATH_FN int xt_rem_pio2(double x, double *rh, double *rl) {
 /* sin(rh + rl), |rh| <= pi/4 (1+eps), |rl| <= ulp(rh).
    sin(rh+rl) = rh + rh^3 S(z) + rl (1 - z/2) + O(rl^2), z = rh^2,
    S(z) = -1/3! + z/5! - ... + z^8/19!  (truncation < 2^-70 relative) */
-XT_MATH_FN double xt_kernel_sin(double rh, double rl) {
-    double z = rh * rh;
+XT_MATH_FN double xt_sin_poly(double z) {
     double p = -XT_IF19;
     p = XT_FMA(p, z, XT_IF17);
     p = XT_FMA(p, z, -XT_IF15);
@@ -230,15 +229,18 @@ XT_MATH_FN double xt_kernel_sin(double rh, double rl) {
     p = XT_FMA(p, z, XT_IF9);
     p = XT_FMA(p, z, -XT_IF7);
     p = XT_FMA(p, z, XT_IF5);
-    p = XT_FMA(p, z, -XT_IF3);
-    double corr = XT_FMA(rh * z, p, rl - 0.5 * z * rl);
+    return XT_FMA(p, z, -XT_IF3);
+}
+
+XT_MATH_FN double xt_kernel_sin(double rh, double rl) {
+    double z = rh * rh;
+    double corr = XT_FMA(rh * z, xt_sin_poly(z), rl - 0.5 * z * rl);
     return rh + corr;
 }
 
 /* cos(rh + rl) = 1 - z/2 + z^2 C(z) - rh rl + O(rl^2),
    C(z) = 1/4! - z/6! + ... + z^9/22! */
-XT_MATH_FN double xt_kernel_cos(double rh, double rl) {
-    double z = rh * rh;
+XT_MATH_FN double xt_cos_poly(double z) {
     double p = XT_IF22;
     p = XT_FMA(p, z, -XT_IF20);
     p = XT_FMA(p, z, XT_IF18);
@@ -248,7 +250,12 @@ XT_MATH_FN double xt_kernel_cos(double rh, double rl) {
     p = XT_FMA(p, z, XT_IF10);
     p = XT_FMA(p, z, -XT_IF8);
     p = XT_FMA(p, z, XT_IF6);
-    p = XT_FMA(p, z, -XT_IF4);
+    return XT_FMA(p, z, -XT_IF4);
+}
+
+XT_MATH_FN double xt_kernel_cos(double rh, double rl) {
+    double z = rh * rh;
+    double p = xt_cos_poly(z);
     /* w = 1 - z/2 with its rounding error recovered (z/2 <= 0.31) */
     double hz = 0.5 * z;
     double w = 1.0 - hz;
@@ -256,6 +263,20 @@ XT_MATH_FN double xt_kernel_cos(double rh, double rl) {
     double tail = XT_FMA(z * z, -p, werr - rh * rl);
     /* note: C(z) above has the opposite sign convention; p = -C(z) */
     return w + tail;
+}
+
+/* xt_sin and xt_cos of 0 < |x| <= pi/4: the kernels with rl = 0, whose terms
+   in rl are then zeros added to non-zero numbers */
+XT_MATH_FN double xt_sin_small(double x) {
+    double z = x * x;
+    return x + x * z * xt_sin_poly(z);
+}
+XT_MATH_FN double xt_cos_small(double x) {
+    double z = x * x;
+    double hz = 0.5 * z;
+    double w = 1.0 - hz;
+    double werr = (1.0 - w) - hz;
+    return w + XT_FMA(z * z, -xt_cos_poly(z), werr);
 }
 
 /* sin and cos of x from one reduction */

@@ -65,8 +65,12 @@ enum { KF_P1 = 1, KF_P2 = 2, KF_P3 = 4, KF_HL = 8, KF_G0 = 16, KF_H1 = 32 };
    and are read and written there (PRef); at_element is not held at all:
    every element passed adds one, so it is a per-particle base plus the
    element index (track_particle). */
-/* slots of the energy fields in PState::slow */
-enum { XS_DELTA = 0, XS_RPP = 1, XS_RVV = 2, XS_INV_RVV = 3, XS_S = 4, XS_ZETA0 = 5, XS_N = 6 };
+/* slots of the energy fields in PState::slow; the compiled code's loop
+   (xt_fast.h) also hands the coordinates to the general code through slots */
+enum {
+    XS_DELTA = 0, XS_RPP = 1, XS_RVV = 2, XS_INV_RVV = 3, XS_S = 4, XS_ZETA0 = 5,
+    XS_X = 6, XS_PX = 7, XS_Y = 8, XS_PY = 9, XS_ZETA = 10, XS_N = 11
+};
 /* dynamic LDS bytes per thread that a tracking kernel launch must provide */
 constexpr int XT_LDS_BYTES_PER_THREAD = XS_N * 8;
 
@@ -1375,8 +1379,8 @@ XT_HD void feature_record(const xtm_features &F, const int64_t i, const double x
    at_element: the reference adds 1 after every element the particle
    survives and sets 0 at the end of a turn; here at_element = base + e at
    element e, with base updated at the end of each turn.
-   run(p, m, run.key(e), c) tracks element e: the program interpreter, or
-   the line's generated code.
+   run(p, m, run.key(e), c) tracks element e: the program interpreter (the
+   compiled code's loop is track_particle_units in xt_fast.h).
    CHI1: the particle's chi is exactly 1.0 and the element code sees the
    constant, so products with chi fold away (chi * k == k exactly) instead
    of being evaluated, or hoisted out of the loops as per-particle values
@@ -1426,27 +1430,12 @@ XT_HD void track_particle_loop(const xtm_particles &P, int64_t i, const Runner &
                current element's arithmetic */
             typename Runner::Key key{};
             if (ele_start < ele_stop) key = run.key(ele_start);
-            for (int64_t e = ele_start; e < ele_stop;) {
-                /* a runner with segments tracks a run of n consecutive
-                   elements in one call (not with element-by-element
-                   records) and returns the position j in the run of the
-                   element where the particle was lost */
-                int64_t n = 1, j = 0;
-                if constexpr (Runner::kSegments) {
-                    const int32_t span = Runner::span(key);
-                    if (span > 1 && flag_monitor != 2 && e + span <= ele_stop) n = span;
-                }
-                const typename Runner::Key next = run.key(e + n < ele_stop ? e + n : e);
+            for (int64_t e = ele_start; e < ele_stop; e++) {
+                const typename Runner::Key next = run.key(e + 1 < ele_stop ? e + 1 : e);
                 if (flag_monitor == 2) XT_MONITOR_RECORD(base + e);
-                if constexpr (Runner::kSegments) {
-                    if (n > 1) j = run.segment(p, m, key, c, e);
-                    else run(p, m, key, c);
-                } else {
-                    run(p, m, key, c);
-                }
+                run(p, m, key, c);
                 if (c.freeze_long()) p.zeta = p.get(XS_ZETA0);
-                if (p.state <= 0) { e_lost = e + j; break; }
-                e += n;
+                if (p.state <= 0) { e_lost = e; break; }
                 key = next;
             }
             if (e_lost >= 0) break;
@@ -1499,7 +1488,6 @@ struct ProgramRunner {
     const int64_t *__restrict__ entry;
     const double *__restrict__ prog;
     using Key = int64_t;
-    static constexpr bool kSegments = false;
     XT_HD Key key(int64_t e) const { return cptr(entry)[e]; }
     XT_HD void operator()(PState<double> &p, const PRef &m, Key pc, const TrackCtx &c) const {
         run_element(p, m, cptr(prog), uniform(pc), c);
@@ -1540,22 +1528,6 @@ XT_HD void track_particle_with(const xtm_particles &P, int64_t i, const Runner1 
     else
         track_particle_loop_cold<false>(P, i, run_other, c, num_turns, ele_start, num_ele_track,
                                         flag_end_turn_actions, flag_reset_s, flag_monitor, mon);
-}
-
-/* The compiled line kernel's body: forward tracking of the particles with
-   chi == 1 only; the interpreter kernel, launched after it on the same
-   stream with skip_chi1 set, tracks the others.  Keeping the interpreter
-   out of this kernel keeps its register allocation and its scratch frame
-   to those of the generated code. */
-template <class Runner1>
-XT_HD void track_particle_chi1(const xtm_particles &P, int64_t i, const Runner1 &run_chi1,
-                               const TrackCtx &c, int32_t num_turns, int32_t ele_start,
-                               int32_t num_ele_track, int32_t flag_end_turn_actions,
-                               int32_t flag_reset_s, int32_t flag_monitor,
-                               const MonRef &mon) {
-    if (!(P.state[i] > 0) || !(P.chi[i] == 1.0)) return;
-    track_particle_loop<true, false>(P, i, run_chi1, c, num_turns, ele_start, num_ele_track,
-                                     flag_end_turn_actions, flag_reset_s, flag_monitor, mon);
 }
 
 /* entry: the forward or, when flags hold XS_FLAG_BACKTRACK, the
