@@ -1,13 +1,14 @@
 """The compiled code's common path (xt_fast.h) on the host against the
 oracle, bit for bit, at the edges of its forms and guards; the statements
-behind its exact quotients at small precisions."""
+behind its exact quotients at small precisions; the cut into segments."""
 import numpy as np
 import pytest
 
 import xtrack_amd as xt
 from fast_path_cases import CASES, IDS, edge_particles
 from helpers import compare_exact, random_particles
-from oracle_backend import GeneratedHostBackend, OracleBackend
+from oracle_backend import GeneratedHostBackend, OracleBackend, generated_host_line
+from xtrack_amd.elements import build_raw_table
 
 
 def _both(make, p, **kw):
@@ -132,3 +133,16 @@ def test_quotient_by_a_number_next_to_one(p):
                 wante = wante + 1          # den = B 2^-p, t = T 2^-(p-1)
             d, _ = _add(q1[0], q1[1], -wantm, wante)
             assert not d.any(), (side, k)
+
+
+def test_segments_follow_the_period():
+    """300 thin elements of period six are cut into ten equal segments, a
+    ring with an irregular element every 31 into two kinds."""
+    from xtrack_amd import lattices
+    for line, kinds, span in ((lattices.thin_fodo_ring(), 1, 30),
+                              (lattices.sextupole_fodo_ring(), 2, 31)):
+        t, o, pp = build_raw_table(line.elements)
+        _, key, _, _, _ = generated_host_line(t, o, pp, line.get_length())
+        spans, seg = (key >> 11) & 31, key >> 16
+        assert seg.max() == kinds
+        assert set(spans[seg > 0]) == {span} and (seg > 0).sum() == 10

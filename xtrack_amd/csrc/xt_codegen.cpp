@@ -50,6 +50,7 @@ constexpr int kSmallCost = 12;
 constexpr size_t kSegMax = 31;           // elements per segment (< 32)
 constexpr int64_t kSegMaxCount = 256;    // distinct segments per line
 constexpr int64_t kSegMaxBody = 2048;    // sum of their lengths
+constexpr int64_t kSegOnceBody = 512;    // the same with segments used once
 // line code: every record literal up to this many distinct records, else
 // literal only for records used more than once whose structure occurs with
 // at most kLiteralPerStruct constant sets, at most kLiteralMax of them
@@ -726,8 +727,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
 
     // Segments: runs of consecutive cheap literal records (drifts,
     // apertures, thin kicks, markers) cut into chunks of at most kSegMax
-    // elements; each chunk sequence that occurs at least twice in the set
-    // becomes one function that tracks the chunk's elements in order and
+    // elements; a chunk sequence becomes one function that tracks the chunk's elements in order and
     // returns the position of the element where the particle was lost.  The
     // key of a chunk's first element carries the segment number and the
     // chunk length; the loop runs the chunk with one dispatch instead of one
@@ -735,47 +735,96 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     // of the single-record path.  (Cheap records are literal: their code
     // reads no constants through rp, which the segment call passes for the
     // chunk's first element only.)
-    std::vector<std::tuple<size_t, size_t, size_t>> chunks;   // (line, first element, length)
-    for (size_t l = 0; l < nl; l++) {
-        const std::vector<int32_t> &rv = recs[l];
-        size_t e = 0;
-        while (e < rv.size()) {
-            if (!cs.small[rv[e]]) { e++; continue; }
-            size_t f = e;
-            while (f < rv.size() && cs.small[rv[f]]) f++;
-            for (size_t a = e; a < f; a += kSegMax) {
-                const size_t n = std::min<size_t>(kSegMax, f - a);
-                if (n > 1) chunks.emplace_back(l, a, n);
+    //
+    // Where a run is cut decides how often its chunks repeat: pieces of a
+    // fixed length suit a run whose period divides it (five cells of six
+    // elements), pieces that begin at one record suit runs with irregular
+    // parts between like cells.  Lengths and the most frequent records are
+    // tried on the whole set, and the cut that leaves the fewest
+    // dispatches is kept.  Chunks that occur once are kept only up to
+    // kSegOnceBody elements of code.
+    using Chunk = std::tuple<size_t, size_t, size_t>;   // (line, first element, length)
+    auto cut = [&](size_t len, int32_t head) {
+        std::vector<Chunk> out;
+        for (size_t l = 0; l < nl; l++) {
+            const std::vector<int32_t> &rv = recs[l];
+            size_t e = 0;
+            while (e < rv.size()) {
+                if (!cs.small[rv[e]]) { e++; continue; }
+                size_t f = e;
+                while (f < rv.size() && cs.small[rv[f]]) f++;
+                while (e < f) {
+                    size_t n = 1;
+                    while (e + n < f && n < len && rv[e + n] != head) n++;
+                    if (n > 1) out.emplace_back(l, e, n);
+                    e += n;
+                }
             }
-            e = f;
         }
-    }
-    using Chunk = std::tuple<size_t, size_t, size_t>;
+        return out;
+    };
     auto chunk_seq = [&](const Chunk &ch) {
         const std::vector<int32_t> &rv = recs[std::get<0>(ch)];
         return std::vector<int32_t>(rv.begin() + std::get<1>(ch),
                                     rv.begin() + std::get<1>(ch) + std::get<2>(ch));
     };
-    std::map<std::vector<int32_t>, int64_t> count;
+    using Ranked = std::vector<std::pair<int64_t, std::vector<int32_t>>>;
+    // the segments of a cut, best first, and the dispatches that they save
+    auto choose = [&](const std::vector<Chunk> &chunks, Ranked &kept) {
+        std::map<std::vector<int32_t>, int64_t> count;
+        for (auto &ch : chunks) count[chunk_seq(ch)]++;
+        Ranked rank;
+        for (auto &kv : count)
+            rank.emplace_back((kv.second - (kv.second > 1 ? 0 : 1)) * (int64_t)kv.first.size(),
+                              kv.first);
+        std::stable_sort(rank.begin(), rank.end(), [](const auto &x, const auto &y) {
+            return x.first > y.first || (x.first == y.first && x.second.size() > y.second.size());
+        });
+        int64_t body = 0, saved = 0;
+        kept.clear();
+        for (auto &r : rank) {
+            const int64_t n = (int64_t)r.second.size(), uses = count[r.second];
+            if ((int64_t)kept.size() >= kSegMaxCount ||
+                body + n > (uses > 1 ? kSegMaxBody : kSegOnceBody))
+                continue;
+            body += n;
+            saved += uses * (n - 1);
+            kept.push_back(r);
+        }
+        // among equal savings, less code
+        return saved * 4096 - body;
+    };
+    std::map<int32_t, int64_t> small_uses;
+    int64_t n_small = 0;
+    for (auto &rv : recs)
+        for (int32_t r : rv)
+            if (cs.small[r]) {
+                small_uses[r]++;
+                n_small++;
+            }
+    std::vector<std::pair<int64_t, int32_t>> heads;
+    for (auto &kv : small_uses) heads.emplace_back(-kv.second, kv.first);
+    std::sort(heads.begin(), heads.end());
+    if (heads.size() > 16) heads.resize(16);
+    std::vector<Chunk> chunks;
+    Ranked seg_rank;
+    int64_t best = -1;
+    auto attempt = [&](size_t len, int32_t head) {
+        std::vector<Chunk> c = cut(len, head);
+        Ranked kept;
+        const int64_t v = choose(c, kept);
+        if (v > best) {
+            best = v;
+            chunks = std::move(c);
+            seg_rank = std::move(kept);
+        }
+    };
+    int64_t tries = 4000000 / std::max<int64_t>(n_small, 1);   // bounds the search for long lines
+    attempt(kSegMax, -1);
+    for (size_t k = 0; k < heads.size() && tries-- > 0; k++) attempt(kSegMax, heads[k].second);
+    for (size_t len = kSegMax - 1; len >= 8 && tries-- > 0; len--) attempt(len, -1);
     std::map<std::vector<int32_t>, Chunk> where;
-    for (auto &ch : chunks) {
-        count[chunk_seq(ch)]++;
-        where.emplace(chunk_seq(ch), ch);
-    }
-    std::vector<std::pair<int64_t, std::vector<int32_t>>> ranked_segs, seg_rank;
-    for (auto &kv : count)
-        if (kv.second >= 2)
-            ranked_segs.emplace_back(kv.second * (int64_t)(kv.first.size() - 1), kv.first);
-    std::stable_sort(ranked_segs.begin(), ranked_segs.end(),
-                     [](const auto &x, const auto &y) { return x.first > y.first; });
-    int64_t seg_body = 0;
-    for (auto &r : ranked_segs) {
-        if ((int64_t)seg_rank.size() >= kSegMaxCount ||
-            seg_body + (int64_t)r.second.size() > kSegMaxBody)
-            continue;
-        seg_body += (int64_t)r.second.size();
-        seg_rank.push_back(r);
-    }
+    for (auto &ch : chunks) where.emplace(chunk_seq(ch), ch);
     std::map<std::vector<int32_t>, int32_t> seg_id;
     for (auto &r : seg_rank) {
         seg_id.emplace(r.second, (int32_t)cs.segs.size());
