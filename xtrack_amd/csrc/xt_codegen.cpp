@@ -209,7 +209,7 @@ struct FastGen {
     const bool loads;
     std::string out;
     bool direct = false;   // holds an op that only the general code has
-    bool clear = false;    // ends with ax = ay = 0
+    bool axay = false;     // sets ax and ay
 
     FastGen(const std::vector<double> &p, bool l) : prog(p), loads(l) {}
 
@@ -489,7 +489,6 @@ struct FastGen {
                 return true;
             }
         }
-        axay = false;
         for (size_t k = 0; k < ops.size(); k++) {
             if (count && k == first) {
                 flush_limits();
@@ -506,12 +505,8 @@ struct FastGen {
                 k = first + period * count - 1;
             }
         }
-        // an entry edge without its exit leaves its own ax, ay
-        if (axay) direct = true;
         return true;
     }
-
-    bool axay = false;
 
     bool emit(int64_t pc) {
         const int64_t op = wbits(prog[pc]);
@@ -555,10 +550,13 @@ struct FastGen {
         case OP_KICK:
             if (!kick(pc)) return false;
             break;
-        case OP_EDGE_AXAY: axay = true; break;
+        case OP_EDGE_AXAY:
+            line("xt::f_edge_axay(p" + cs(a, 2) + ");");
+            axay = true;
+            break;
         case OP_EDGE_CLEAR_AXAY:
-            axay = false;
-            clear = true;
+            line("p.ax = p.ay = 0.;");
+            axay = true;
             break;
         case OP_EDGE_LINEAR:
             if (!loads && prog[a] == 0.0 && prog[a + 1] == 0.0) {
@@ -604,7 +602,7 @@ struct FastGen {
     std::string body() {
         flush_limits();
         if (direct) return "    p.bad = true;\n";
-        if (clear) line("p.clear = true;");
+        if (axay) line("p.axay = true;");
         return out;
     }
 };
@@ -955,15 +953,18 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
 
 }  // namespace
 
-int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector<double> &prog,
-                            int32_t waves_per_eu, uint32_t options, std::string &src,
-                            std::vector<int32_t> &rec_of_elem, std::string &err) {
+namespace {
+
+int line_source(const std::vector<int64_t> &entry, const std::vector<double> &prog,
+                int32_t waves_per_eu, uint32_t options, std::string &src,
+                std::vector<int32_t> &rec_of_elem, std::string &err, bool backtrack) {
     CodeSet cs;
     std::vector<std::vector<int32_t>> recs;
     const int st = build_code_set({&entry}, {&prog}, false, cs, recs, err);
     if (st != XTM_OK) return st;
     rec_of_elem = std::move(recs[0]);
     std::string s = emit_code_set(cs, options, "line code");
+    const std::string bt = backtrack ? "<true>" : "<false>";
     s += "}  // namespace xt_gen\n\n";
     s += "#if defined(__HIPCC__)\n";
     char occ[128];
@@ -976,12 +977,12 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
          "    int32_t num_turns, int32_t ele_start, int32_t num_ele_track,\n"
          "    int32_t flag_end_turn_actions, int32_t flag_reset_s, int32_t flag_monitor,\n"
          "    const xtm_monitor *__restrict__ Md, const xtm_particles *__restrict__ Pd,\n"
-         "    uint64_t flags) {\n"
+         "    uint64_t flags, int32_t num_ele_line) {\n"
          "    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;\n"
-         "    const xt::TrackCtx c{flags, line_length, P.q0, P.t_sim};\n"
+         "    const xt::TrackCtx c{flags, line_length, P.q0, P.t_sim, num_ele_line};\n"
          "    // chi == 1 particles; the interpreter kernel tracks the others\n"
          "    const bool alive = i < P.capacity && P.state[i] > 0 && P.chi[i] == 1.0;\n"
-         "    xt::track_particle_units(P, i, alive, xt_gen::Runner{rec, entry, prog}, c,\n"
+         "    xt::track_particle_units" + bt + "(P, i, alive, xt_gen::Runner{rec, entry, prog}, c,\n"
          "                             num_turns, ele_start, num_ele_track,\n"
          "                             flag_end_turn_actions, flag_reset_s, flag_monitor,\n"
          "                             xt::MonRef{Md, Pd});\n"
@@ -992,13 +993,16 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
          "    double line_length, const xtm_particles *P, int32_t num_turns, int32_t ele_start,\n"
          "    int32_t num_ele_track, int32_t flag_end_turn_actions, int32_t flag_reset_s,\n"
          "    int32_t flag_monitor, const xtm_monitor *M, uint64_t flags) {\n"
-         "    xtm_monitor m0 = {};\n"
-         "    const xt::TrackCtx c{flags, line_length, P->q0, P->t_sim};\n"
+         "    xtm_monitor m0 = {};\n" +
+         (backtrack ? std::string("    const int64_t num_ele_line = ") +
+                          std::to_string(entry.size()) + ";\n"
+                    : std::string("    const int64_t num_ele_line = 0;\n")) +
+         "    const xt::TrackCtx c{flags, line_length, P->q0, P->t_sim, num_ele_line};\n"
          "    const xt::MonRef mon{M ? M : &m0, P};\n"
          "    for (int64_t i = 0; i < P->capacity; i++) {\n"
          "        if (!(P->state[i] > 0)) continue;\n"
          "        if (P->chi[i] == 1.0)\n"
-         "            xt::track_particle_units(*P, i, true, xt_gen::Runner{rec, entry, prog}, c,\n"
+         "            xt::track_particle_units" + bt + "(*P, i, true, xt_gen::Runner{rec, entry, prog}, c,\n"
          "                                     num_turns, ele_start, num_ele_track,\n"
          "                                     flag_end_turn_actions, flag_reset_s,\n"
          "                                     flag_monitor, mon);\n"
@@ -1012,6 +1016,21 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
          "#endif\n";
     src = std::move(s);
     return XTM_OK;
+}
+
+}  // namespace
+
+int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector<double> &prog,
+                            int32_t waves_per_eu, uint32_t options, std::string &src,
+                            std::vector<int32_t> &rec_of_elem, std::string &err) {
+    return line_source(entry, prog, waves_per_eu, options, src, rec_of_elem, err, false);
+}
+
+int xt_generate_backtrack_source(const std::vector<int64_t> &entry,
+                                 const std::vector<double> &prog, int32_t waves_per_eu,
+                                 std::string &src, std::vector<int32_t> &rec_of_elem,
+                                 std::string &err) {
+    return line_source(entry, prog, waves_per_eu, 0, src, rec_of_elem, err, true);
 }
 
 
@@ -1046,7 +1065,7 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "    // chi == 1 particles; the interpreter batch kernel tracks the others\n"
          "    const bool alive = (int32_t)threadIdx.x < b.count && P.state[i] > 0 &&\n"
          "                       P.chi[i] == 1.0;\n"
-         "    xt::track_particle_units(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
+         "    xt::track_particle_units<false>(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
          "                             xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
          "                             num_turns, 0, (int32_t)ne, 1, 1, 0,\n"
          "                             xt::MonRef{nullptr, Pd});\n"
@@ -1065,7 +1084,7 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "        for (int64_t i = b.first; i < b.first + b.count; i++) {\n"
          "            if (!(P->state[i] > 0)) continue;\n"
          "            if (P->chi[i] == 1.0)\n"
-         "                xt::track_particle_units(*P, i, true,\n"
+         "                xt::track_particle_units<false>(*P, i, true,\n"
          "                    xt_gen::Runner{recs[b.line], entries[b.line], progs[b.line]}, c,\n"
          "                    num_turns, 0, (int32_t)ne, 1, 1, 0, mon);\n"
          "            else\n"

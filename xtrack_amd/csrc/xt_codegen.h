@@ -33,6 +33,13 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
                             int32_t waves_per_eu, uint32_t options, std::string &src,
                             std::vector<int32_t> &rec_of_elem, std::string &err);
 
+// The same for tracking backwards: `entry` holds the backtracking programs in
+// reverse element order, in which the kernel also counts its elements.
+int xt_generate_backtrack_source(const std::vector<int64_t> &entry,
+                                 const std::vector<double> &prog, int32_t waves_per_eu,
+                                 std::string &src, std::vector<int32_t> &rec_of_elem,
+                                 std::string &err);
+
 // Source of a translation unit that tracks a batch of lines in one launch:
 // one function per distinct element structure (the record code with its
 // constants read from the line's program at rp = prog + entry[e], so that

@@ -47,9 +47,10 @@ namespace xt {
 struct FState {
     double x, px, y, py, zeta, s;
     double delta, rpp, rvv, inv_rvv;
+    double ax, ay;   /* of the last magnet edge; stored late (axay) */
     /* bad: outside a range; out, outg: outside a local aperture, outside
-       the global limit; clear: the unit ends with ax = ay = 0 */
-    bool bad, out, outg, clear;
+       the global limit; axay: the unit sets ax and ay */
+    bool bad, out, outg, axay;
     uint32_t ones;   /* all ones: a case that f_polar leaves out was met */
 };
 
@@ -330,6 +331,11 @@ XT_HD void f_edge_linear(FState &p, const double r21, const double r43) {
     p.py = p.py + r43 * p.y;
 }
 
+XT_HD void f_edge_axay(FState &p, const double ca, const double cb) {
+    p.ax = ca * (p.y - 0.0);
+    p.ay = cb * (p.x - 0.0);
+}
+
 XT_HD void f_xy_shift(FState &p, const double ax, const double ay) {
     p.x = p.x + ax;
     p.y = p.y + ay;
@@ -390,13 +396,12 @@ XT_HD double *thread_slots(double *host_slots, int32_t *stride) {
    the unit's first element.  A lost particle is stored, with the element of
    the unit where it was lost; returns false for it.
    Out of line: its registers and calls take no part in the common path. */
-template <class Runner>
+template <bool BT, class Runner>
 XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key key,
                                       double *host_slots, const int64_t i, const MonRef mon,
                                       const uint64_t flags, const double line_length,
                                       const int32_t e, const int32_t n, const int64_t at_turn,
                                       const int64_t at_element, const bool record) {
-    constexpr bool BT = false;
     const xtm_particles &P = *mon.P;
     const TrackCtx c{flags, line_length, P.q0, P.t_sim, 0};
     PState<double> p;
@@ -421,7 +426,7 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
         P.x[i] = p.x; P.px[i] = p.px; P.y[i] = p.y; P.py[i] = p.py;
         P.zeta[i] = p.zeta; P.delta[i] = p.delta();
         P.rpp[i] = p.rpp(); P.rvv[i] = p.rvv(); P.s[i] = p.s();
-        P.at_element[i] = at_element + j;
+        P.at_element[i] = BT ? at_element - j : at_element + j;
         P.at_turn[i] = at_turn; P.state[i] = p.state;
         return false;
     }
@@ -430,18 +435,14 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
     return true;
 }
 
-/* ax = ay = 0 (the exit edge of a bend), out of line */
-XT_HD_COLD void clear_axay(const xtm_particles *P, const int64_t i) {
-    P->ax[i] = 0.;
-    P->ay[i] = 0.;
-}
-
-/* One particle with chi == 1 through [ele_start, ele_start + num_ele_track)
-   for num_turns turns, forward (track_particle_loop of xt_ops.h with the
-   units of the file comment).  All lanes of a wave walk the units together;
-   a lane without a particle, or whose particle is lost, takes part without
-   effect (alive false), so that the loops are scalar. */
-template <class Runner>
+/* One particle with chi == 1 through num_ele_track elements from ele_start
+   for num_turns turns (track_particle_loop of xt_ops.h with the units of the
+   file comment).  BT: backtracking; the runner's elements are then the line's
+   in reverse order with their backtracking programs, and ele_start counts in
+   that order.  All lanes of a wave walk the units together; a lane without a
+   particle, or whose particle is lost, takes part without effect (alive
+   false), so that the loops are scalar. */
+template <bool BT, class Runner>
 XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool alive,
                                 const Runner &run, const TrackCtx &c, const int32_t num_turns,
                                 const int32_t ele_start, const int32_t num_ele_track,
@@ -456,14 +457,14 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
     int32_t stride;
     double *slot = thread_slots(host_slots, &stride);
     FState p = {};
-    int64_t at_turn = 0, base = 0;
+    int64_t at_turn = 0, at_el = 0;   /* at_el: at_element at ele_start */
     if (alive) {
         p.x = P.x[i]; p.px = P.px[i]; p.y = P.y[i]; p.py = P.py[i];
         p.zeta = P.zeta[i]; p.s = P.s[i];
         p.delta = P.delta[i]; p.rpp = P.rpp[i]; p.rvv = P.rvv[i];
         p.inv_rvv = 1. / p.rvv;
         at_turn = P.at_turn[i];
-        base = P.at_element[i] - ele_start;   /* at_element = base + e at element e */
+        at_el = P.at_element[i];
         slot[XS_DELTA * stride] = p.delta;
         slot[XS_RPP * stride] = p.rpp;
         slot[XS_RVV * stride] = p.rvv;
@@ -472,16 +473,25 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
     }
     const int32_t ele_stop = ele_start + num_ele_track;
     bool e_ok = f_energy_ok(p.delta, p.rpp, p.rvv, p.inv_rvv);
-    bool clean = false;   /* ax = ay = 0 stored since the last general unit */
+    bool axay = false;    /* p.ax and p.ay are not stored yet */
 
+    auto store_axay = [&]() {
+        if (axay && alive) {
+            mon.P->ax[i] = p.ax;
+            mon.P->ay[i] = p.ay;
+        }
+        axay = false;
+    };
     /* the general code on the unit; false when the particle is lost */
     auto general = [&](FState &q, const typename Runner::Key key, const int32_t e,
                        const int32_t n, const bool record) {
         slot[XS_X * stride] = p.x; slot[XS_PX * stride] = p.px;
         slot[XS_Y * stride] = p.y; slot[XS_PY * stride] = p.py;
         slot[XS_ZETA * stride] = p.zeta; slot[XS_S * stride] = p.s;
-        const bool kept = track_unit_general(run, key, host_slots, i, mon, c.flags,
-                                             c.line_length, e, n, at_turn, base + e, record);
+        const int64_t k = e - ele_start;
+        const bool kept = track_unit_general<BT>(run, key, host_slots, i, mon, c.flags,
+                                                 c.line_length, e, n, at_turn,
+                                                 BT ? at_el - k : at_el + k, record);
         q.x = slot[XS_X * stride]; q.px = slot[XS_PX * stride];
         q.y = slot[XS_Y * stride]; q.py = slot[XS_PY * stride];
         q.zeta = slot[XS_ZETA * stride]; q.s = slot[XS_S * stride];
@@ -491,11 +501,17 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
     };
 
     for (int32_t iturn = 0; iturn < num_turns; iturn++) {
+        if (BT && flag_end_turn_actions > 0) {
+            at_turn -= 1;
+            at_el = c.num_ele_line;
+            if (flag_reset_s > 0) p.s = c.line_length;
+        }
         typename Runner::Key key{};
         if (ele_start < ele_stop) key = run.key(ele_start);
-        if (flag_monitor == 1 && alive) {
+        if (!BT && flag_monitor == 1) {
+            store_axay();
             FState q = p;
-            general(q, key, ele_start, 0, true);
+            if (alive) general(q, key, ele_start, 0, true);
         }
         for (int32_t e = ele_start; e < ele_stop;) {
             int32_t n = 1;
@@ -504,7 +520,7 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
             const typename Runner::Key next = run.key(e + n < ele_stop ? e + n : e);
             FState q = p;
             q.bad = !e_ok;
-            q.out = q.outg = q.clear = false;
+            q.out = q.outg = q.axay = false;
             q.ones = 0;
             if (flag_monitor == 2) q.bad = true;
             else if (n > 1) run.fast_segment(q, key);
@@ -514,38 +530,41 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
             if (c.freeze_long()) q.zeta = slot[XS_ZETA0 * stride];
             q.bad &= alive;
             if (__builtin_expect(wave_any(q.bad), 0)) {
+                store_axay();
                 if (q.bad) {
                     alive = general(q, key, e, n, flag_monitor == 2);
                     e_ok = f_energy_ok(q.delta, q.rpp, q.rvv, q.inv_rvv);
+                } else if (q.axay && alive) {
+                    mon.P->ax[i] = q.ax;
+                    mon.P->ay[i] = q.ay;
                 }
-                clean = false;
                 if (!wave_any(alive)) return;
-            }
-            if (q.clear && !clean) {
-                if (alive) clear_axay(mon.P, i);
-                clean = true;
+            } else {
+                axay |= q.axay;
             }
             p = q;
             e += n;
             key = next;
         }
-        if (flag_monitor == 2 && alive) {
+        if (flag_monitor == 2) {
+            store_axay();
             FState q = p;
-            general(q, key, ele_stop, 0, true);
+            if (alive) general(q, key, ele_stop, 0, true);
         }
-        if (flag_end_turn_actions > 0) {
+        if (!BT && flag_end_turn_actions > 0) {
             at_turn += 1;
-            base = -(int64_t)ele_start;
+            at_el = 0;
             if (flag_reset_s > 0) p.s = 0.;
         } else {
-            base += num_ele_track;
+            at_el += BT ? -num_ele_track : num_ele_track;
         }
     }
+    store_axay();
     if (alive) {
         P.x[i] = p.x; P.px[i] = p.px; P.y[i] = p.y; P.py[i] = p.py;
         P.zeta[i] = p.zeta; P.delta[i] = p.delta;
         P.rpp[i] = p.rpp; P.rvv[i] = p.rvv; P.s[i] = p.s;
-        P.at_element[i] = base + ele_start;
+        P.at_element[i] = at_el;
         P.at_turn[i] = at_turn;
     }
 }

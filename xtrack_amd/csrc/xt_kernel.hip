@@ -170,6 +170,22 @@ int32_t hip_fail(hipError_t e, const char *where) {
    files (matrix products) */
 int32_t xt_report_error(int32_t code, const char *msg) { return fail(code, msg); }
 
+/* Generated code of a line on its device: the kernel, the element keys and
+   the entry offsets in the order in which the kernel counts elements. */
+struct LineCode {
+    int32_t *d_rec = nullptr;
+    int64_t *d_entry = nullptr;
+    hipModule_t module = nullptr;
+    hipFunction_t kernel = nullptr;
+
+    void release() {
+        if (d_rec) (void)hipFree(d_rec);
+        if (d_entry) (void)hipFree(d_entry);
+        if (module) (void)hipModuleUnload(module);
+        *this = LineCode();
+    }
+};
+
 struct xtm_line {
     int32_t device;
     int64_t num_elements;
@@ -186,10 +202,12 @@ struct xtm_line {
     xtm_particles *d_mon_p = nullptr;
     xtm_monitor *d_mon_m = nullptr;
     // generated line code (xtm_line_specialize)
-    int32_t *d_rec = nullptr;
-    hipModule_t module = nullptr;
-    hipFunction_t kernel = nullptr;
+    LineCode code;
     uint32_t spec_options = 0;
+    // the same for backtracking (backtrack_code): compiled on first use
+    std::mutex bt_mutex;
+    LineCode bt;
+    int32_t bt_waves = 0;      // occupancy target; 0: no compiled code wanted
 };
 
 struct xtm_batch {
@@ -360,16 +378,58 @@ int32_t xtm_line_destroy(xtm_line *L) {
     if (L->d_entry) (void)hipFree(L->d_entry);
     if (L->d_entry_bt) (void)hipFree(L->d_entry_bt);
     if (L->d_prog) (void)hipFree(L->d_prog);
-    if (L->d_rec) (void)hipFree(L->d_rec);
     if (L->d_mon_p) (void)hipFree(L->d_mon_p);
     if (L->d_mon_m) (void)hipFree(L->d_mon_m);
-    if (L->module) (void)hipModuleUnload(L->module);
+    L->code.release();
+    L->bt.release();
     delete L;
     return XTM_OK;
 }
 
 int32_t xtm_line_specialize(xtm_line *L, int32_t waves_per_eu) {
     return xtm_line_specialize_ex(L, waves_per_eu, 0);
+}
+
+/* Line code of the programs `entry` (in tracking order), loaded on the
+   line's device. */
+static int32_t load_line_code(const xtm_line *L, const std::vector<int64_t> &entry,
+                              int32_t waves_per_eu, uint32_t options, bool backtrack,
+                              LineCode &out) {
+    std::string src, err;
+    std::vector<int32_t> rec;
+    if (L->num_elements > 0x7fffffff)
+        return fail(XTM_ERR_UNSUPPORTED, "xtm_line_specialize: line too long");
+    int st = backtrack
+                 ? xt_generate_backtrack_source(entry, L->prog, waves_per_eu, src, rec, err)
+                 : xt_generate_line_source(entry, L->prog, waves_per_eu, options, src, rec, err);
+    if (st != XTM_OK) return fail(st, "xtm_line_specialize: " + err);
+    std::vector<char> code;
+    st = rtc_compile(src, code);
+    if (st != XTM_OK) return st;
+    hipError_t e = hipSetDevice(L->device);
+    if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
+    LineCode c;
+    auto failed = [&](const char *what) {
+        c.release();
+        return hip_fail(e, what);
+    };
+    if ((e = hipModuleLoadData(&c.module, code.data())) != hipSuccess)
+        return hip_fail(e, "hipModuleLoadData");
+    if ((e = hipModuleGetFunction(&c.kernel, c.module, "xtm_line_kernel")) != hipSuccess)
+        return failed("hipModuleGetFunction");
+    const size_t nr = rec.empty() ? 1 : rec.size();
+    if ((e = hipMalloc(&c.d_rec, nr * sizeof(int32_t))) != hipSuccess ||
+        (e = hipMalloc(&c.d_entry, nr * sizeof(int64_t))) != hipSuccess)
+        return failed("hipMalloc");
+    if (!rec.empty() &&
+        ((e = hipMemcpy(c.d_rec, rec.data(), rec.size() * sizeof(int32_t),
+                        hipMemcpyHostToDevice)) != hipSuccess ||
+         (e = hipMemcpy(c.d_entry, entry.data(), entry.size() * sizeof(int64_t),
+                        hipMemcpyHostToDevice)) != hipSuccess))
+        return failed("hipMemcpy");
+    out.release();
+    out = c;
+    return XTM_OK;
 }
 
 int32_t xtm_line_specialize_ex(xtm_line *L, int32_t waves_per_eu, uint32_t options) {
@@ -381,49 +441,41 @@ int32_t xtm_line_specialize_ex(xtm_line *L, int32_t waves_per_eu, uint32_t optio
     if (waves_per_eu < 0 || waves_per_eu > 8)
         return fail(XTM_ERR_ARG, "xtm_line_specialize: waves_per_eu outside 0..8");
     if (waves_per_eu == 0) waves_per_eu = XTM_COMPILED_WAVES_PER_EU;
-    std::string src, err;
-    std::vector<int32_t> rec;
-    int st = xt_generate_line_source(L->entry, L->prog, waves_per_eu, options, src, rec, err);
-    if (st != XTM_OK) return fail(st, "xtm_line_specialize: " + err);
-    std::vector<char> code;
-    st = rtc_compile(src, code);
+    const int32_t st = load_line_code(L, L->entry, waves_per_eu, options, false, L->code);
     if (st != XTM_OK) return st;
-    hipError_t e = hipSetDevice(L->device);
-    if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
-    hipModule_t mod = nullptr;
-    if ((e = hipModuleLoadData(&mod, code.data())) != hipSuccess)
-        return hip_fail(e, "hipModuleLoadData");
-    hipFunction_t fn = nullptr;
-    if ((e = hipModuleGetFunction(&fn, mod, "xtm_line_kernel")) != hipSuccess) {
-        (void)hipModuleUnload(mod);
-        return hip_fail(e, "hipModuleGetFunction");
-    }
-    int32_t *d_rec = nullptr;
-    const size_t nr = rec.empty() ? 1 : rec.size();
-    if ((e = hipMalloc(&d_rec, nr * sizeof(int32_t))) != hipSuccess) {
-        (void)hipModuleUnload(mod);
-        return hip_fail(e, "hipMalloc");
-    }
-    if (!rec.empty() &&
-        (e = hipMemcpy(d_rec, rec.data(), rec.size() * sizeof(int32_t),
-                       hipMemcpyHostToDevice)) != hipSuccess) {
-        (void)hipFree(d_rec);
-        (void)hipModuleUnload(mod);
-        return hip_fail(e, "hipMemcpy");
-    }
-    if (L->d_rec) (void)hipFree(L->d_rec);
-    if (L->module) (void)hipModuleUnload(L->module);
-    L->d_rec = d_rec;
-    L->module = mod;
-    L->kernel = fn;
     L->spec_options = options;
+    std::lock_guard<std::mutex> lk(L->bt_mutex);
+    L->bt_waves = waves_per_eu;
     return XTM_OK;
 }
 
-int32_t xtm_line_is_specialized(const xtm_line *L) { return (L && L->kernel) ? 1 : 0; }
+/* The compiled backtracking code of a compiled line, compiled on its first
+   use (a line is rarely tracked backwards, and the code takes as long as the
+   forward code to compile); nullptr: the interpreter tracks instead (the line
+   is not compiled, its backtracking programs do not compile, or the first use
+   is inside a stream capture, where nothing can be loaded).  Always in exact
+   arithmetic.  Collider ring, 100,003 particles, one turn back: 81.7 ms with
+   the interpreter, 12.8 ms. */
+static const LineCode *backtrack_code(xtm_line *L, hipStream_t stream) {
+    if (!L->code.kernel) return nullptr;
+    std::lock_guard<std::mutex> lk(L->bt_mutex);
+    if (L->bt.kernel) return &L->bt;
+    if (L->bt_waves == 0) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+        return nullptr;
+    const std::vector<int64_t> rev(L->entry_bt.rbegin(), L->entry_bt.rend());
+    if (load_line_code(L, rev, L->bt_waves, 0, true, L->bt) != XTM_OK) {
+        L->bt_waves = 0;
+        return nullptr;
+    }
+    return &L->bt;
+}
+
+int32_t xtm_line_is_specialized(const xtm_line *L) { return (L && L->code.kernel) ? 1 : 0; }
 
 int32_t xtm_line_specialized_options(const xtm_line *L) {
-    return (L && L->kernel) ? (int32_t)L->spec_options : -1;
+    return (L && L->code.kernel) ? (int32_t)L->spec_options : -1;
 }
 
 int32_t xtm_line_generate_source(const xtm_line *L, int32_t waves_per_eu, char *buf,
@@ -506,38 +558,35 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
     const int64_t nblocks = (P->capacity + BLOCK - 1) / BLOCK;
     if (nblocks > 0x7fffffff) return fail(XTM_ERR_ARG, "too many particles");
     const bool backtrack = (track_flags >> XTM_FLAG_BACKTRACK) & 1;
-    if (L->kernel && !backtrack) {
+    const LineCode *code = backtrack ? backtrack_code(L, (hipStream_t)stream)
+                           : L->code.kernel ? &L->code : nullptr;
+    if (code) {
         xtm_particles Pv = *P;
-        const int32_t *rec = L->d_rec;
-        const int64_t *entry = L->d_entry;
+        const int32_t *rec = code->d_rec;
+        const int64_t *entry = code->d_entry;
         const double *prog = L->d_prog;
         double line_length = L->line_length;
-        int32_t a_turns = num_turns, a_start = ele_start, a_n = num_ele_track;
+        int32_t a_turns = num_turns, a_n = num_ele_track;
+        int32_t a_nele = (int32_t)L->num_elements;
+        // backtracking code counts the elements from the line's end
+        int32_t a_start = backtrack ? a_nele - ele_start - num_ele_track : ele_start;
         int32_t a_end = flag_end_turn_actions, a_reset = flag_reset_s_at_end_turn;
         int32_t a_mon = flag_monitor;
         uint64_t a_flags = track_flags;
         void *args[] = {&rec, &entry, &prog, &line_length, &Pv, &a_turns, &a_start, &a_n,
-                        &a_end, &a_reset, &a_mon, &Md, &Pd, &a_flags};
-        e = hipModuleLaunchKernel(L->kernel, (unsigned)nblocks, 1, 1, BLOCK, 1, 1, kLdsLine,
+                        &a_end, &a_reset, &a_mon, &Md, &Pd, &a_flags, &a_nele};
+        e = hipModuleLaunchKernel(code->kernel, (unsigned)nblocks, 1, 1, BLOCK, 1, 1, kLdsLine,
                                   (hipStream_t)stream, args, nullptr);
         if (e != hipSuccess) return hip_fail(e, "xtm_line_kernel launch");
-        /* particles with chi != 1 on the interpreter, same stream */
-        hipLaunchKernelGGL(track_kernel, dim3((unsigned)nblocks), dim3(BLOCK), kLdsLine,
-                           (hipStream_t)stream, L->d_entry, L->d_prog, L->line_length,
-                           (int64_t)L->num_elements, Pd, num_turns, ele_start, num_ele_track,
-                           flag_end_turn_actions, flag_reset_s_at_end_turn, flag_monitor, Md,
-                           track_flags, (int32_t)1);
-        e = hipGetLastError();
-        if (e != hipSuccess) return hip_fail(e, "track_kernel launch");
-        return XTM_OK;
     }
-    /* backtracking always runs on the interpreter, with the backtracking
-       programs */
+    /* the interpreter: every particle, or after the compiled code those with
+       chi != 1, on the same stream */
     hipLaunchKernelGGL(track_kernel, dim3((unsigned)nblocks), dim3(BLOCK), kLdsLine,
                        (hipStream_t)stream, backtrack ? L->d_entry_bt : L->d_entry, L->d_prog,
                        L->line_length, (int64_t)L->num_elements, Pd,
                        num_turns, ele_start, num_ele_track, flag_end_turn_actions,
-                       flag_reset_s_at_end_turn, flag_monitor, Md, track_flags, (int32_t)0);
+                       flag_reset_s_at_end_turn, flag_monitor, Md, track_flags,
+                       (int32_t)(code ? 1 : 0));
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "track_kernel launch");
     return XTM_OK;

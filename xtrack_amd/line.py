@@ -62,8 +62,9 @@ class Line:
         order, so coordinates match the reference's arithmetic bit for bit
         given the same elementary functions; 'fast' (compiled code only)
         re-associates the sector-bend polar drift onto reciprocals with a few
-        ulp of error per element.  Particles with chi != 1 and backtracking
-        always run the exact interpreter."""
+        ulp of error per element.  Particles with chi != 1 always run the
+        interpreter; backtracking always runs in exact arithmetic, compiled
+        on its first use when the line is compiled."""
         dev = device or (_context if isinstance(_context, str) else None) or 'cuda:0'
         self.tracker = Tracker(self, backend=backend, device=dev, compile=compile,
                                waves_per_eu=waves_per_eu, arithmetic=arithmetic)
