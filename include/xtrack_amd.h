@@ -477,6 +477,20 @@ int32_t xtm_gemm_bf16_noalloc(const uint16_t *A, int64_t sam, int64_t sak, const
                               void *stream);
 int64_t xtm_gemm_bf16_scratch_floats(void);
 
+/* The 16-256-256-256-1 network (ReLU between the layers) on M rows in one
+ * kernel, the activations in registers: out[r] = f((x[r] - mean) / std), times
+ * y_std plus y_mean when `scale` is set; mean (and std) may be NULL for x as it
+ * is.  x: M x 16 FP32, row-major, 16-byte aligned; w, b: host arrays of the
+ * four layers' device pointers (w[k] in x out row-major, FP32, rounded to BF16
+ * here); workspace: xtm_mlp_workspace_bytes() bytes of device memory, 16-byte
+ * aligned, written on `stream`.  The same bits as the four products through
+ * xtm_gemm_bf16. */
+int64_t xtm_mlp_workspace_bytes(void);
+int32_t xtm_mlp_forward(const float *x, const float *mean, const float *std,
+                        const float *const *w, const float *const *b, void *workspace,
+                        float *out, int64_t M, int32_t scale, float y_std, float y_mean,
+                        void *stream);
+
 /* Wait for all work queued on `stream`. */
 int32_t xtm_synchronize(void *stream);
 

@@ -278,6 +278,236 @@ int32_t gemm_check(const uint16_t *A, const uint16_t *B, const float *C, int64_t
     return XTM_OK;
 }
 
+/* ---- the 16-256-256-256-1 network in one kernel ------------------------------
+ *
+ * Layer by layer through xtm_gemm_bf16 a prediction moves every activation
+ * through HBM in FP32 and BF16: 262,147 rows took 0.99 ms.  Here the
+ * activations stay in registers from the input to the output: 0.076 ms, 940
+ * TFLOP/s (a large BF16 library product on this card: 1230).
+ *
+ * The products run transposed, Z^T = W^T H^T: weights are the A operand (rows:
+ * output features), activations the B operand (columns: batch rows), so that a
+ * lane's results belong to its own batch column.  The accumulator of a
+ * 16-feature tile holds features 4 (l / 16) + j of column l % 16 in lane l; the
+ * next layer's B operand wants features 8 (l / 16) + j, j < 8, of a 32-feature
+ * step.  Two tiles a, b of one step become that operand by swapping the lower
+ * half of b with the upper half of a and then the odd rows of 16 lanes of one
+ * with the even rows of the other: 2 swaps per 32-bit word, no LDS.  Every
+ * k step multiplies the same 32 features in the same places as
+ * gemm_bf16_kernel, steps in order, so the results are the same bits.
+ *
+ * A wave carries MLP_CT = 3 column tiles (48 batch rows): with 4 tiles the two
+ * layers' operands alone are 256 registers; with 3 a wave stays within 256 and
+ * two blocks share a CU.  A weight fragment (1 KB) read from LDS serves 3
+ * products of 16 cycles: 85 bytes per clock and CU, of 128.  Weights come
+ * packed in fragment order and pass through LDS in chunks of 64 features (32
+ * KB), the next chunk copied by global_load_lds while this one multiplies. */
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int MLP_H = 256;                       // hidden width
+constexpr int MLP_IN = 16;
+constexpr int MLP_CT = 3;                        // column tiles per wave
+constexpr int MLP_ROWS = 4 * 16 * MLP_CT;        // batch rows per block
+constexpr int MLP_FRAG = 1024;                   // bytes of one 16 x 32 fragment
+constexpr int MLP_CHUNK = 32 * MLP_FRAG;         // 64 features x 256 inputs
+// packed weights in bytes: layer 1 (16 tiles x 1 step), 2 and 3 (16 x 8),
+// 4 (1 x 8), then the biases (3 x 256 + 1 floats)
+constexpr int MLP_P1 = 0, MLP_P2 = 16 * MLP_FRAG, MLP_P3 = MLP_P2 + 128 * MLP_FRAG,
+              MLP_P4 = MLP_P3 + 128 * MLP_FRAG, MLP_PB = MLP_P4 + 8 * MLP_FRAG,
+              MLP_PACKED = MLP_PB + (3 * MLP_H + 4) * 4;
+
+struct MlpWeights {
+    const float *w[4];   // [in][out] row-major
+    const float *b[4];
+};
+
+/* Packed fragments: fragment (tile t, step s) of a layer holds, for lane l and
+   j < 8, W[k = 32 s + 8 (l / 16) + j][n = 16 t + l % 16] in BF16 (zero outside
+   the layer).  One thread per lane and fragment; 280 fragments. */
+__global__ __launch_bounds__(256) void mlp_pack_kernel(MlpWeights W, unsigned char *out) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    const int f = idx >> 6, lane = idx & 63;
+    if (f < 280) {
+        int layer, t, st;
+        if (f < 16) { layer = 0; t = f; st = 0; }
+        else if (f < 144) { layer = 1; t = (f - 16) >> 3; st = (f - 16) & 7; }
+        else if (f < 272) { layer = 2; t = (f - 144) >> 3; st = (f - 144) & 7; }
+        else { layer = 3; t = 0; st = f - 272; }
+        const int K = layer == 0 ? MLP_IN : MLP_H, N = layer == 3 ? 1 : MLP_H;
+        const int n = 16 * t + (lane & 15), k0 = 32 * st + 8 * (lane >> 4);
+        u16x8 v;
+        for (int j = 0; j < 8; j++)
+            v[j] = (k0 + j < K && n < N)
+                       ? f32_to_bf16_rne(W.w[layer][(int64_t)(k0 + j) * N + n])
+                       : (uint16_t)0;
+        *reinterpret_cast<u16x8 *>(out + (int64_t)f * MLP_FRAG + lane * 16) = v;
+    } else {
+        const int k = idx - 280 * 64;
+        float *bo = reinterpret_cast<float *>(out + MLP_PB);
+        if (k < 3 * MLP_H) bo[k] = W.b[k >> 8][k & 255];
+        else if (k == 3 * MLP_H) bo[k] = W.b[3][0];
+    }
+}
+
+/* `bytes` (a multiple of 4096) from global memory into LDS, 16 bytes a lane,
+   asynchronous: complete after the next s_waitcnt vmcnt(0) and barrier */
+__device__ __forceinline__ void copy_to_lds(const unsigned char *src, unsigned char *dst,
+                                            int bytes) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int o = wave * 1024; o < bytes; o += 4096)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void *)(src + o + lane * 16),
+            (__attribute__((address_space(3))) void *)(dst + o), 16, 0, 0);
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    bf16x2 v;
+    v[0] = (__bf16)a;
+    v[1] = (__bf16)b;
+    uint32_t u;
+    __builtin_memcpy(&u, &v, 4);
+    return u;
+}
+
+__device__ __forceinline__ void swap_tiles(uint32_t &a, uint32_t &b) {
+    u32x2 r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    r = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+    a = r[0];
+    b = r[1];
+}
+
+/* One 32-feature step p of a hidden layer (tiles 2p, 2p + 1): products over
+   STEPS k steps, bias, ReLU, BF16, and the next layer's operand of the step. */
+template <int STEPS>
+__device__ __forceinline__ void mlp_step(const unsigned char *frag, const float *bias,
+                                         const bf16x8 (&in)[STEPS][MLP_CT],
+                                         bf16x8 (&out)[MLP_CT], int lane) {
+    f32x4 acc[2][MLP_CT];
+    for (int t = 0; t < 2; t++)
+        for (int c = 0; c < MLP_CT; c++) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const bf16x8 w = *reinterpret_cast<const bf16x8 *>(
+                frag + (t * STEPS + s) * MLP_FRAG + lane * 16);
+#pragma unroll
+            for (int c = 0; c < MLP_CT; c++)
+                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, in[s][c], acc[t][c], 0, 0, 0);
+        }
+    uint32_t h[2][MLP_CT][2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const f32x4 b = *reinterpret_cast<const f32x4 *>(&bias[16 * t + 4 * (lane >> 4)]);
+#pragma unroll
+        for (int c = 0; c < MLP_CT; c++) {
+            float v[4];
+            for (int j = 0; j < 4; j++) {
+                v[j] = acc[t][c][j] + b[j];
+                if (!(v[j] > 0.f)) v[j] = 0.f;
+            }
+            h[t][c][0] = pack_bf16(v[0], v[1]);
+            h[t][c][1] = pack_bf16(v[2], v[3]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < MLP_CT; c++) {
+        swap_tiles(h[0][c][0], h[1][c][0]);
+        swap_tiles(h[0][c][1], h[1][c][1]);
+        const u32x4 u = {h[0][c][0], h[0][c][1], h[1][c][0], h[1][c][1]};
+        __builtin_memcpy(&out[c], &u, 16);
+    }
+}
+
+/* out[r] = network((x[r] - mean) / std) * y_std + y_mean for r < M (mean
+   nullptr: x as it is; scale 0: without y_std and y_mean) */
+__global__ __launch_bounds__(256, 2) void mlp_forward_kernel(
+    const float *__restrict__ x, const float *__restrict__ mean, const float *__restrict__ std,
+    const unsigned char *__restrict__ packed, float *__restrict__ out, int64_t M, int32_t scale,
+    float y_std, float y_mean) {
+    __shared__ __align__(16) unsigned char wbuf[2][MLP_CHUNK];
+    __shared__ __align__(16) float bias[3 * MLP_H + 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, g = lane >> 4;
+    const int64_t row0 = (int64_t)blockIdx.x * MLP_ROWS + wave * 16 * MLP_CT + col;
+    copy_to_lds(packed + MLP_P1, wbuf[0], 16 * MLP_FRAG);
+    for (int k = threadIdx.x; k < 3 * MLP_H + 1; k += 256)
+        bias[k] = reinterpret_cast<const float *>(packed + MLP_PB)[k];
+    // the input operand: features 8 g + j of batch row row0 + 16 c, one step,
+    // zero from feature 16 on
+    bf16x8 x0[1][MLP_CT];
+#pragma unroll
+    for (int c = 0; c < MLP_CT; c++) {
+        const int64_t row = row0 + 16 * c;
+        float v[8];
+        for (int j = 0; j < 8; j++) v[j] = 0.f;
+        if (g < 2 && row < M) {
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(&x[row * MLP_IN + 8 * g]);
+            const f32x4 b = *reinterpret_cast<const f32x4 *>(&x[row * MLP_IN + 8 * g + 4]);
+            for (int j = 0; j < 4; j++) {
+                v[j] = a[j];
+                v[j + 4] = b[j];
+            }
+            if (mean)
+                for (int j = 0; j < 8; j++) v[j] = (v[j] - mean[8 * g + j]) / std[8 * g + j];
+        }
+        for (int j = 0; j < 8; j++) x0[0][c][j] = (__bf16)v[j];
+    }
+    bf16x8 h1[8][MLP_CT], h2[8][MLP_CT];
+    int buf = 0;
+    auto next = [&](const unsigned char *src, int bytes) {
+        // the chunk copied last is complete, and the other buffer is free
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (bytes) copy_to_lds(src, wbuf[buf ^ 1], bytes);
+    };
+    next(packed + MLP_P2, MLP_CHUNK);
+#pragma unroll
+    for (int p = 0; p < 8; p++)
+        mlp_step<1>(wbuf[buf] + 2 * p * MLP_FRAG, bias + 32 * p, x0, h1[p], lane);
+    buf ^= 1;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        next(q < 3 ? packed + MLP_P2 + (q + 1) * MLP_CHUNK : packed + MLP_P3, MLP_CHUNK);
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+            mlp_step<8>(wbuf[buf] + 16 * p * MLP_FRAG, bias + MLP_H + 64 * q + 32 * p, h1,
+                        h2[2 * q + p], lane);
+        buf ^= 1;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        next(q < 3 ? packed + MLP_P3 + (q + 1) * MLP_CHUNK : packed + MLP_P4,
+             q < 3 ? MLP_CHUNK : 8 * MLP_FRAG);
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+            mlp_step<8>(wbuf[buf] + 16 * p * MLP_FRAG, bias + 2 * MLP_H + 64 * q + 32 * p, h2,
+                        h1[2 * q + p], lane);
+        buf ^= 1;
+    }
+    next(nullptr, 0);
+    f32x4 acc[MLP_CT];
+    for (int c = 0; c < MLP_CT; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        const bf16x8 w =
+            *reinterpret_cast<const bf16x8 *>(wbuf[buf] + s * MLP_FRAG + lane * 16);
+#pragma unroll
+        for (int c = 0; c < MLP_CT; c++)
+            acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, h1[s][c], acc[c], 0, 0, 0);
+    }
+    // feature 0 of every column lies in the first 16 lanes
+    if (g == 0)
+        for (int c = 0; c < MLP_CT; c++) {
+            const int64_t row = row0 + 16 * c;
+            float v = acc[c][0] + bias[3 * MLP_H];
+            if (scale) v = v * y_std + y_mean;
+            if (row < M) out[row] = v;
+        }
+}
+
 /* workspace of xtm_gemm_bf16: allocated once per device on first need */
 constexpr int kMaxDevices = 64;
 std::mutex g_ws_mutex;
@@ -354,5 +584,37 @@ int32_t xtm_gemm_bf16_noalloc(const uint16_t *A, int64_t sam, int64_t sak, const
 }
 
 int64_t xtm_gemm_bf16_scratch_floats(void) { return GEMM_WS_FLOATS; }
+
+int64_t xtm_mlp_workspace_bytes(void) { return MLP_PACKED; }
+
+int32_t xtm_mlp_forward(const float *x, const float *mean, const float *std,
+                        const float *const *w, const float *const *b, void *workspace,
+                        float *out, int64_t M, int32_t scale, float y_std, float y_mean,
+                        void *stream) {
+    if (!x || !w || !b || !workspace || !out || M < 0 || (mean && !std) ||
+        ((uintptr_t)x & 15) || ((uintptr_t)workspace & 15))
+        return xt_report_error(XTM_ERR_ARG, "xtm_mlp_forward: null or misaligned argument");
+    MlpWeights W;
+    for (int k = 0; k < 4; k++) {
+        if (!w[k] || !b[k])
+            return xt_report_error(XTM_ERR_ARG, "xtm_mlp_forward: null weights");
+        W.w[k] = w[k];
+        W.b[k] = b[k];
+    }
+    if (M == 0) return XTM_OK;
+    const int64_t nb = (M + MLP_ROWS - 1) / MLP_ROWS;
+    if (nb > 0x7fffffff) return xt_report_error(XTM_ERR_ARG, "xtm_mlp_forward: too many rows");
+    unsigned char *packed = static_cast<unsigned char *>(workspace);
+    const int threads = 280 * 64 + 3 * MLP_H + 1;
+    hipLaunchKernelGGL(mlp_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, W, packed);
+    if (hipGetLastError() != hipSuccess)
+        return xt_report_error(XTM_ERR_HIP, "xtm_mlp_forward: kernel launch failed");
+    hipLaunchKernelGGL(mlp_forward_kernel, dim3((unsigned)nb), dim3(256), 0,
+                       (hipStream_t)stream, x, mean, std, packed, out, M, scale, y_std, y_mean);
+    return hipGetLastError() == hipSuccess
+               ? XTM_OK
+               : xt_report_error(XTM_ERR_HIP, "xtm_mlp_forward: kernel launch failed");
+}
 
 }  // extern "C"

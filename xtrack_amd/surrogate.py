@@ -113,8 +113,38 @@ class MLP:
         self.x_mean = self.x_std = None
         self.y_mean, self.y_std = 0.0, 1.0
 
+    def _one_kernel(self, x, *vectors):
+        """Whether xtm_mlp_forward takes x: this network's sizes, FP32
+        throughout, on one device; everything else goes layer by layer."""
+        torch = _t()
+        ts = [x, *vectors, *self.W, *self.b]
+        return (self.sizes == SIZES and x.dim() == 2 and x.shape[1] == SIZES[0] and len(x) > 0
+                and all(t.dtype == torch.float32 and t.device == x.device for t in ts)
+                and x.is_cuda and all(t.is_contiguous() for t in self.W + self.b)
+                and all(tuple(t.shape) == (SIZES[0],) for t in vectors)
+                and [tuple(w.shape) for w in self.W] == list(zip(SIZES[:-1], SIZES[1:]))
+                and [tuple(b.shape) for b in self.b] == [(n,) for n in SIZES[1:]])
+
+    def _run_one_kernel(self, x, mean=None, std=None, y_std=None, y_mean=None):
+        torch = _t()
+        lib = _native.load()
+        x = x.contiguous()
+        if x.data_ptr() % 16:
+            x = x.clone()
+        if mean is not None:
+            mean, std = mean.contiguous(), std.contiguous()
+        out = torch.empty(len(x), dtype=torch.float32, device=x.device)
+        work = torch.empty(lib.xtm_mlp_workspace_bytes(), dtype=torch.uint8, device=x.device)
+        ptrs = [(ctypes.c_void_p * 4)(*[t.data_ptr() for t in v]) for v in (self.W, self.b)]
+        _native.check(lib.xtm_mlp_forward(
+            _ptr(x), _ptr(mean), _ptr(std), ptrs[0], ptrs[1], _ptr(work), _ptr(out), len(x),
+            int(y_std is not None), y_std or 0.0, y_mean or 0.0, _stream(x.device)))
+        return out
+
     def forward(self, x, keep=False):
         """x: (B, 16) FP32 on the device (already normalised)."""
+        if not keep and self._one_kernel(x):
+            return self._run_one_kernel(x)
         h = to_bf16(x)
         acts = [h]
         zs = []
@@ -235,6 +265,8 @@ class MLP:
 
     def predict(self, x, batch=65536):
         torch = _t()
+        if self._one_kernel(x, self.x_mean, self.x_std):
+            return self._run_one_kernel(x, self.x_mean, self.x_std, self.y_std, self.y_mean)
         xn = (x - self.x_mean) / self.x_std
         out = [self.forward(xn[s:s + batch]) for s in range(0, len(xn), batch)]
         return torch.cat(out) * self.y_std + self.y_mean
