@@ -491,6 +491,29 @@ int32_t xtm_mlp_forward(const float *x, const float *mean, const float *std,
                         float *out, int64_t M, int32_t scale, float y_std, float y_mean,
                         void *stream);
 
+/* A training step of an n-layer network sizes[0]-...-sizes[n] (n <= 8, ReLU
+ * between the layers, sizes[n] = 1) on B rows, without an allocation beyond
+ * xtm_gemm_bf16's workspace; the same products as through xtm_gemm_bf16.
+ * forward: xb B x sizes[0] in BF16; w, b: host arrays of device pointers (FP32,
+ * w[l] sizes[l] x sizes[l + 1]); wb: scratch for all weights in BF16; z and h:
+ * the hidden layers' outputs one after the other, FP32 and BF16; out: B.
+ * backward: dout = d loss / d out (B, FP32) to the gradients gw[l], gb[l]; dz
+ * and dzb: scratch of the size of z, and of h plus B. */
+int32_t xtm_mlp_train_forward(int32_t n, const int64_t *sizes, const uint16_t *xb,
+                              const float *const *w, const float *const *b, uint16_t *wb,
+                              float *z, uint16_t *h, float *out, int64_t B, void *stream);
+int32_t xtm_mlp_train_backward(int32_t n, const int64_t *sizes, const uint16_t *xb,
+                               const uint16_t *h, const float *z, const float *const *w,
+                               const float *dout, uint16_t *wb, float *dz, uint16_t *dzb,
+                               float *const *gw, float *const *gb, int64_t B, void *stream);
+
+/* One Adam update of n <= 16 FP32 arrays of count[k] values in place: *t (device)
+ * is the step count, this step included; alpha = 1 - beta. */
+int32_t xtm_adam_step(int32_t n, float *const *p, const float *const *g, float *const *m,
+                      float *const *v, const int64_t *count, const float *t, float lr,
+                      float beta1, float alpha1, float beta2, float alpha2, float eps,
+                      void *stream);
+
 /* Wait for all work queued on `stream`. */
 int32_t xtm_synchronize(void *stream);
 

@@ -211,6 +211,13 @@ def load():
     lib.xtm_mlp_forward.argtypes = [c.c_void_p, c.c_void_p, c.c_void_p, c.c_void_p, c.c_void_p,
                                     c.c_void_p, c.c_void_p, c.c_int64, c.c_int32, c.c_float,
                                     c.c_float, c.c_void_p]
+    lib.xtm_mlp_train_forward.restype = c.c_int32
+    lib.xtm_mlp_train_forward.argtypes = [c.c_int32] + [c.c_void_p] * 8 + [c.c_int64, c.c_void_p]
+    lib.xtm_mlp_train_backward.restype = c.c_int32
+    lib.xtm_mlp_train_backward.argtypes = [c.c_int32] + [c.c_void_p] * 11 + [c.c_int64,
+                                                                           c.c_void_p]
+    lib.xtm_adam_step.restype = c.c_int32
+    lib.xtm_adam_step.argtypes = [c.c_int32] + [c.c_void_p] * 6 + [c.c_float] * 6 + [c.c_void_p]
     lib.xtm_synchronize.restype = c.c_int32
     lib.xtm_synchronize.argtypes = [c.c_void_p]
     lib.xtm_math_eval.restype = c.c_int32

@@ -115,8 +115,8 @@ __device__ __forceinline__ void store_tile(uint16_t *S, const u16x8 v, int64_t s
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(
     const uint16_t *__restrict__ A, int64_t sam, int64_t sak, const uint16_t *__restrict__ B,
     int64_t sbk, int64_t sbn, float *__restrict__ C, int64_t ldc, uint16_t *__restrict__ Cb,
-    const float *__restrict__ bias, int32_t relu, int64_t M, int64_t N, int64_t K, int64_t kc,
-    float *__restrict__ ws) {
+    const float *__restrict__ bias, int32_t relu, const float *__restrict__ mask, int64_t M,
+    int64_t N, int64_t K, int64_t kc, float *__restrict__ ws) {
     // operand tiles during the k loop, the result tile after it
     __shared__ __align__(16) unsigned char smem[TM * CLD * 4];
     uint16_t *As = reinterpret_cast<uint16_t *>(smem);
@@ -188,6 +188,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(
             for (int e = 0; e < 4; e++) {
                 if (bias && n + e < N) v[e] += bias[n + e];
                 if (relu && !(v[e] > 0.f)) v[e] = 0.f;
+                if (mask && n + e < N) v[e] *= mask[m * ldc + n + e] > 0.f ? 1.f : 0.f;
             }
         }
         if (vec && n + 4 <= N) {
@@ -211,8 +212,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(
 /* Sum of the `splits` partial tiles in split order, then the epilogue. */
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(
     const float *__restrict__ ws, int64_t splits, float *__restrict__ C, int64_t ldc,
-    uint16_t *__restrict__ Cb, const float *__restrict__ bias, int32_t relu, int64_t M,
-    int64_t N) {
+    uint16_t *__restrict__ Cb, const float *__restrict__ bias, int32_t relu,
+    const float *__restrict__ mask, int64_t M, int64_t N) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= M * N) return;
     const int64_t m = e / N, n = e % N;
@@ -220,6 +221,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(
     for (int64_t s = 0; s < splits; s++) v += ws[s * M * N + e];
     if (bias) v += bias[n];
     if (relu && !(v > 0.f)) v = 0.f;
+    if (mask) v *= mask[m * ldc + n] > 0.f ? 1.f : 0.f;
     C[m * ldc + n] = v;
     if (Cb) Cb[m * ldc + n] = f32_to_bf16_rne(v);
 }
@@ -243,7 +245,7 @@ int32_t gemm_launch(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t 
                     int64_t sbk, int64_t sbn, float *C, int64_t ldc, uint16_t *Cb,
                     const float *bias, int32_t relu, int64_t M, int64_t N, int64_t K,
                     hipStream_t stream, float *ws, int64_t ws_floats, int64_t splits,
-                    int64_t kc) {
+                    int64_t kc, const float *mask = nullptr) {
     const int64_t gy = (M + TM - 1) / TM, gx = (N + TN - 1) / TN;
     if (splits > 1) {
         if (!ws || splits * M * N > ws_floats)
@@ -251,16 +253,16 @@ int32_t gemm_launch(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t 
                                                 "workspace");
         hipLaunchKernelGGL(gemm_bf16_kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)splits),
                            dim3(256), 0, stream, A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias,
-                           relu, M, N, K, kc, ws);
+                           relu, mask, M, N, K, kc, ws);
         if (hipGetLastError() != hipSuccess)
             return xt_report_error(XTM_ERR_HIP, "xtm_gemm_bf16: kernel launch failed");
         const int64_t nb = (M * N + 255) / 256;
         hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)nb), dim3(256), 0, stream, ws,
-                           splits, C, ldc, Cb, bias, relu, M, N);
+                           splits, C, ldc, Cb, bias, relu, mask, M, N);
     } else {
         hipLaunchKernelGGL(gemm_bf16_kernel, dim3((unsigned)gx, (unsigned)gy, 1), dim3(256), 0,
-                           stream, A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias, relu, M, N, K,
-                           K > 0 ? K : 1, (float *)nullptr);
+                           stream, A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias, relu, mask, M, N,
+                           K, K > 0 ? K : 1, (float *)nullptr);
     }
     return hipGetLastError() == hipSuccess
                ? XTM_OK
@@ -508,6 +510,82 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_kernel(
         }
 }
 
+/* ---- the training step's elementwise work -----------------------------------
+ * A step on 1,024 rows holds 30 MFLOP of elementwise work on 140,000 weights;
+ * as some 150 tensor operations it took 0.84 ms, all of it launches.  Each
+ * kernel here does one kind of it for every layer at once. */
+constexpr int MLP_MAX = 8;   // layers
+
+struct ConvertList {
+    const float *src[MLP_MAX + 1];
+    uint16_t *dst[MLP_MAX + 1];
+    int64_t end[MLP_MAX + 1];   // running element counts
+    int32_t n;
+};
+
+__global__ __launch_bounds__(256) void convert_kernel(ConvertList L) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int t = 0;
+    while (t < L.n && e >= L.end[t]) t++;
+    if (t == L.n) return;
+    const int64_t k = e - (t ? L.end[t - 1] : 0);
+    L.dst[t][k] = f32_to_bf16_rne(L.src[t][k]);
+}
+
+struct SumList {
+    const float *a[MLP_MAX];
+    float *out[MLP_MAX];
+    int64_t cols[MLP_MAX], block_end[MLP_MAX];
+    int32_t n;
+};
+
+/* Column sums of row-major (rows x cols) arrays: 16 columns per block, 16
+   threads per column over the rows, their partial sums in double. */
+__global__ __launch_bounds__(256) void column_sum_kernel(SumList L, int64_t rows) {
+    __shared__ double part[16][17];
+    int t = 0;
+    while (t + 1 < L.n && (int64_t)blockIdx.x >= L.block_end[t]) t++;
+    const int64_t b0 = t ? L.block_end[t - 1] : 0;
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+    const int64_t col = 16 * ((int64_t)blockIdx.x - b0) + c, n = L.cols[t];
+    double s = 0.0;
+    if (col < n)
+        for (int64_t k = r; k < rows; k += 16) s += (double)L.a[t][k * n + col];
+    part[r][c] = s;
+    __syncthreads();
+    if (r == 0 && col < n) {
+        for (int k = 1; k < 16; k++) s += part[k][c];
+        L.out[t][col] = (float)s;
+    }
+}
+
+struct AdamList {
+    float *p[2 * MLP_MAX], *m[2 * MLP_MAX], *v[2 * MLP_MAX];
+    const float *g[2 * MLP_MAX];
+    int64_t end[2 * MLP_MAX];
+    int32_t n;
+};
+
+/* One Adam update of every weight and bias; *t is the step count, this step
+   included.  Bound by the 28 bytes per weight it moves: 140,000 weights in
+   one launch against 94 tensor operations. */
+__global__ __launch_bounds__(256) void adam_kernel(AdamList L, const float *__restrict__ t,
+                                                   float lr, float beta1, float alpha1,
+                                                   float beta2, float alpha2, float eps) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int k = 0;
+    while (k < L.n && e >= L.end[k]) k++;
+    if (k == L.n) return;
+    const int64_t i = e - (k ? L.end[k - 1] : 0);
+    const float bc1 = 1.f - powf(beta1, *t), bc2 = 1.f - powf(beta2, *t);
+    const float g = L.g[k][i];
+    const float m = fmaf(alpha1, g, L.m[k][i] * beta1);
+    const float v = fmaf(alpha2 * g, g, L.v[k][i] * beta2);
+    L.m[k][i] = m;
+    L.v[k][i] = v;
+    L.p[k][i] -= lr * (m / bc1) / (sqrtf(v / bc2) + eps);
+}
+
 /* workspace of xtm_gemm_bf16: allocated once per device on first need */
 constexpr int kMaxDevices = 64;
 std::mutex g_ws_mutex;
@@ -526,12 +604,12 @@ float *g_scratch[kMaxDevices] = {};
 
 }  // namespace
 
-extern "C" {
+namespace {
 
-int32_t xtm_gemm_bf16(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t *B,
-                      int64_t sbk, int64_t sbn, float *C, int64_t ldc, uint16_t *Cb,
-                      const float *bias, int32_t relu, int64_t M, int64_t N, int64_t K,
-                      void *stream) {
+int32_t gemm_with_workspace(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t *B,
+                            int64_t sbk, int64_t sbn, float *C, int64_t ldc, uint16_t *Cb,
+                            const float *bias, int32_t relu, const float *mask, int64_t M,
+                            int64_t N, int64_t K, hipStream_t stream) {
     int32_t st = gemm_check(A, B, C, ldc, M, N, K);
     if (st != XTM_OK || M == 0 || N == 0) return st;
     int64_t kc;
@@ -548,8 +626,150 @@ int32_t xtm_gemm_bf16(const uint16_t *A, int64_t sam, int64_t sak, const uint16_
         }
         ws = g_ws[dev];
     }
-    return gemm_launch(A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias, relu, M, N, K,
-                       (hipStream_t)stream, ws, GEMM_WS_FLOATS, splits, kc);
+    return gemm_launch(A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias, relu, M, N, K, stream, ws,
+                       GEMM_WS_FLOATS, splits, kc, mask);
+}
+
+int32_t launched(const char *what) {
+    return hipGetLastError() == hipSuccess ? XTM_OK : xt_report_error(XTM_ERR_HIP, what);
+}
+
+/* FP32 -> BF16 of the weights of layers [first, n), into their place in the
+   concatenation of all layers, and of `more` (n_more values) when not null */
+int32_t convert_weights(int32_t first, int32_t n, const int64_t *sizes, const float *const *w,
+                        uint16_t *wb, const float *more, uint16_t *more_b, int64_t n_more,
+                        hipStream_t stream) {
+    ConvertList L;
+    L.n = 0;
+    int64_t total = 0, off = 0;
+    for (int32_t l = 0; l < n; l++) {
+        const int64_t c = sizes[l] * sizes[l + 1];
+        if (l >= first) {
+            L.src[L.n] = w[l];
+            L.dst[L.n] = wb + off;
+            L.end[L.n++] = total += c;
+        }
+        off += c;
+    }
+    if (more) {
+        L.src[L.n] = more;
+        L.dst[L.n] = more_b;
+        L.end[L.n++] = total += n_more;
+    }
+    hipLaunchKernelGGL(convert_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       stream, L);
+    return launched("xtm_mlp_train: kernel launch failed");
+}
+
+bool train_args_ok(int32_t n, const int64_t *sizes, int64_t B) {
+    if (n < 1 || n > MLP_MAX || !sizes || B < 1 || sizes[n] != 1) return false;
+    int64_t total = 0;
+    for (int32_t l = 0; l <= n; l++) {
+        if (sizes[l] < 1 || sizes[l] > 1 << 20) return false;
+        if (l) total += sizes[l - 1] * sizes[l];
+    }
+    return total < (int64_t)1 << 38 && B < (int64_t)1 << 31;
+}
+
+}  // namespace
+
+extern "C" {
+
+int32_t xtm_mlp_train_forward(int32_t n, const int64_t *sizes, const uint16_t *xb,
+                              const float *const *w, const float *const *b, uint16_t *wb,
+                              float *z, uint16_t *h, float *out, int64_t B, void *stream) {
+    if (!train_args_ok(n, sizes, B) || !xb || !w || !b || !wb || !out || (n > 1 && (!z || !h)))
+        return xt_report_error(XTM_ERR_ARG, "xtm_mlp_train_forward: invalid arguments");
+    const hipStream_t s = (hipStream_t)stream;
+    int32_t st = convert_weights(0, n, sizes, w, wb, nullptr, nullptr, 0, s);
+    const uint16_t *in = xb;
+    for (int32_t l = 0; l < n && st == XTM_OK; l++) {
+        const int64_t K = sizes[l], N = sizes[l + 1];
+        const bool last = l == n - 1;
+        st = gemm_with_workspace(in, K, 1, wb, N, 1, last ? out : z, N, last ? nullptr : h, b[l],
+                                 last ? 0 : 1, nullptr, B, N, K, s);
+        in = h;
+        wb += K * N;
+        if (!last) {
+            z += B * N;
+            h += B * N;
+        }
+    }
+    return st;
+}
+
+int32_t xtm_mlp_train_backward(int32_t n, const int64_t *sizes, const uint16_t *xb,
+                               const uint16_t *h, const float *z, const float *const *w,
+                               const float *dout, uint16_t *wb, float *dz, uint16_t *dzb,
+                               float *const *gw, float *const *gb, int64_t B, void *stream) {
+    if (!train_args_ok(n, sizes, B) || !xb || !w || !dout || !wb || !dzb || !gw || !gb ||
+        (n > 1 && (!h || !z || !dz)))
+        return xt_report_error(XTM_ERR_ARG, "xtm_mlp_train_backward: invalid arguments");
+    const hipStream_t s = (hipStream_t)stream;
+    // hidden layer l: z, dz (its first n - 1 layers) and h at off[l]; dzb also
+    // holds the output layer's, at off[n - 1]
+    int64_t off[MLP_MAX + 1] = {0}, woff[MLP_MAX + 1] = {0};
+    for (int32_t l = 0; l < n; l++) {
+        off[l + 1] = off[l] + B * sizes[l + 1];
+        woff[l + 1] = woff[l] + sizes[l] * sizes[l + 1];
+    }
+    int32_t st = convert_weights(1, n, sizes, w, wb, dout, dzb + off[n - 1], B, s);
+    SumList S;
+    S.n = n;
+    int64_t blocks = 0;
+    for (int32_t l = n - 1; l >= 0 && st == XTM_OK; l--) {
+        const int64_t K = sizes[l], N = sizes[l + 1];
+        const uint16_t *d = dzb + off[l], *in = l ? h + off[l - 1] : xb;
+        // h^T dz
+        st = gemm_with_workspace(in, 1, K, d, N, 1, gw[l], N, nullptr, nullptr, 0, nullptr, K, N,
+                                 B, s);
+        if (l > 0 && st == XTM_OK)   // dz W^T where the layer below is active
+            st = gemm_with_workspace(d, N, 1, wb + woff[l], 1, N, dz + off[l - 1], K,
+                                     dzb + off[l - 1], nullptr, 0, z + off[l - 1], B, K, N, s);
+    }
+    if (st != XTM_OK) return st;
+    for (int32_t l = 0; l < n; l++) {
+        S.a[l] = l == n - 1 ? dout : dz + off[l];
+        S.out[l] = gb[l];
+        S.cols[l] = sizes[l + 1];
+        S.block_end[l] = blocks += (sizes[l + 1] + 15) / 16;
+    }
+    hipLaunchKernelGGL(column_sum_kernel, dim3((unsigned)blocks), dim3(256), 0, s, S, B);
+    return launched("xtm_mlp_train_backward: kernel launch failed");
+}
+
+int32_t xtm_adam_step(int32_t n, float *const *p, const float *const *g, float *const *m,
+                      float *const *v, const int64_t *count, const float *t, float lr,
+                      float beta1, float alpha1, float beta2, float alpha2, float eps,
+                      void *stream) {
+    if (n < 1 || n > 2 * MLP_MAX || !p || !g || !m || !v || !count || !t)
+        return xt_report_error(XTM_ERR_ARG, "xtm_adam_step: invalid arguments");
+    AdamList L;
+    int64_t total = 0;
+    L.n = n;
+    for (int32_t k = 0; k < n; k++) {
+        if (!p[k] || !g[k] || !m[k] || !v[k] || count[k] < 0)
+            return xt_report_error(XTM_ERR_ARG, "xtm_adam_step: null array");
+        L.p[k] = p[k];
+        L.g[k] = g[k];
+        L.m[k] = m[k];
+        L.v[k] = v[k];
+        L.end[k] = total += count[k];
+    }
+    if (total == 0) return XTM_OK;
+    if (total > (int64_t)1 << 38)
+        return xt_report_error(XTM_ERR_ARG, "xtm_adam_step: too many values");
+    hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, L, t, lr, beta1, alpha1, beta2, alpha2, eps);
+    return launched("xtm_adam_step: kernel launch failed");
+}
+
+int32_t xtm_gemm_bf16(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t *B,
+                      int64_t sbk, int64_t sbn, float *C, int64_t ldc, uint16_t *Cb,
+                      const float *bias, int32_t relu, int64_t M, int64_t N, int64_t K,
+                      void *stream) {
+    return gemm_with_workspace(A, sam, sak, B, sbk, sbn, C, ldc, Cb, bias, relu, nullptr, M, N,
+                               K, (hipStream_t)stream);
 }
 
 int32_t xtm_gemm_bf16_noalloc(const uint16_t *A, int64_t sam, int64_t sak, const uint16_t *B,

@@ -39,6 +39,10 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
 
 
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
 def _stream(dev):
     torch = _t()
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
@@ -135,16 +139,46 @@ class MLP:
             mean, std = mean.contiguous(), std.contiguous()
         out = torch.empty(len(x), dtype=torch.float32, device=x.device)
         work = torch.empty(lib.xtm_mlp_workspace_bytes(), dtype=torch.uint8, device=x.device)
-        ptrs = [(ctypes.c_void_p * 4)(*[t.data_ptr() for t in v]) for v in (self.W, self.b)]
         _native.check(lib.xtm_mlp_forward(
-            _ptr(x), _ptr(mean), _ptr(std), ptrs[0], ptrs[1], _ptr(work), _ptr(out), len(x),
+            _ptr(x), _ptr(mean), _ptr(std), _pointers(self.W), _pointers(self.b), _ptr(work),
+            _ptr(out), len(x),
             int(y_std is not None), y_std or 0.0, y_mean or 0.0, _stream(x.device)))
         return out
 
     def forward(self, x, keep=False):
         """x: (B, 16) FP32 on the device (already normalised)."""
+        torch = _t()
         if not keep and self._one_kernel(x):
             return self._run_one_kernel(x)
+        if not self._native_step(x) or x.shape[1] != self.sizes[0]:
+            return self._forward_layers(x, keep)
+        lib = _native.load()
+        B = len(x)
+        hidden = B * sum(self.sizes[1:-1])
+        xb = to_bf16(x).contiguous()
+        z = torch.empty(hidden, dtype=torch.float32, device=x.device)
+        h = torch.empty(hidden, dtype=torch.int16, device=x.device)
+        out = torch.empty(B, dtype=torch.float32, device=x.device)
+        wb = self._weight_scratch()
+        _native.check(lib.xtm_mlp_train_forward(
+            len(self.W), self._sizes_array(), _ptr(xb), _pointers(self.W), _pointers(self.b),
+            _ptr(wb), _ptr(z), _ptr(h), _ptr(out), B, _stream(x.device)))
+        if keep:
+            self._cache = (xb, z, h)
+        return out
+
+    def _native_step(self, x):
+        """Whether the library's training step takes this network (at most 8
+        layers, one output, contiguous FP32 parameters) and the rows of x."""
+        torch = _t()
+        ps = self.W + self.b
+        shapes = list(zip(self.sizes[:-1], self.sizes[1:])) + [(n,) for n in self.sizes[1:]]
+        return (len(self.W) <= 8 and self.sizes[-1] == 1 and len(x) > 0 and x.is_cuda
+                and all(p.dtype == torch.float32 and p.device == x.device and p.is_contiguous()
+                        for p in ps) and [tuple(p.shape) for p in ps] == shapes)
+
+    def _forward_layers(self, x, keep):
+        """The forward pass product by product, for any network."""
         h = to_bf16(x)
         acts = [h]
         zs = []
@@ -161,9 +195,8 @@ class MLP:
             self._cache = (acts, zs)
         return zs[-1][:, 0]
 
-    def backward(self, dout):
-        """Gradients of the weights and biases for d(loss)/d(output) =
-        dout (B,), after forward(keep=True)."""
+    def _backward_layers(self, dout):
+        """The backward pass after _forward_layers."""
         acts, zs = self._cache
         n = len(self.W)
         dz = dout.reshape(-1, 1).to(_t().float32)
@@ -177,20 +210,61 @@ class MLP:
                 dz = dh * (zs[li - 1] > 0).to(dh.dtype)
         return gW, gb
 
-    def adam_step(self, gW, gb, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
-        """One Adam update of the weights and biases in place.  The step
-        count and the bias corrections live on the device, so that the update
-        can be captured in a HIP graph and replayed."""
+    def _sizes_array(self):
+        return (ctypes.c_int64 * len(self.sizes))(*self.sizes)
+
+    def _weight_scratch(self):
         torch = _t()
+        n = sum(i * o for i, o in zip(self.sizes[:-1], self.sizes[1:]))
+        return torch.empty(n, dtype=torch.int16, device=self.device)
+
+    def backward(self, dout):
+        """Gradients of the weights and biases for d(loss)/d(output) =
+        dout (B,), after forward(keep=True)."""
+        torch = _t()
+        if len(self._cache) == 2:
+            return self._backward_layers(dout)
+        lib = _native.load()
+        xb, z, h = self._cache
+        B, n = len(xb), len(self.W)
+        dout = dout.reshape(-1).to(torch.float32).contiguous()
+        if len(dout) != B:
+            raise ValueError(f'dout must have the {B} rows of the forward pass')
+        w = self.W
+        gW = [torch.empty_like(t) for t in w]
+        gb = [torch.empty_like(t) for t in self.b]
+        dz = torch.empty_like(z)
+        dzb = torch.empty(len(z) + B, dtype=torch.int16, device=z.device)
+        wb = self._weight_scratch()
+        _native.check(lib.xtm_mlp_train_backward(
+            n, self._sizes_array(), _ptr(xb), _ptr(h), _ptr(z), _pointers(w), _ptr(dout),
+            _ptr(wb), _ptr(dz), _ptr(dzb), _pointers(gW), _pointers(gb), B, _stream(z.device)))
+        return gW, gb
+
+    def adam_step(self, gW, gb, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
+        """One Adam update of the weights and biases in place (FP32 arrays on
+        the device: in one kernel).  The step count lives on the device, so that the update can be captured
+        in a HIP graph and replayed."""
+        torch = _t()
+        params, grads = self.W + self.b, list(gW) + list(gb)
         if self._adam is None:
             self._adam = {'t': torch.zeros((), dtype=torch.float32, device=self.device),
-                          'm': [torch.zeros_like(p) for p in self.W + self.b],
-                          'v': [torch.zeros_like(p) for p in self.W + self.b]}
+                          'm': [torch.zeros_like(p) for p in params],
+                          'v': [torch.zeros_like(p) for p in params]}
         st = self._adam
         st['t'].add_(1.0)
+        if (len(params) <= 16 and len(grads) == len(params) and st['t'].is_cuda
+                and all(t.dtype == torch.float32 and t.device == st['t'].device
+                        and t.is_contiguous() and t.shape == p.shape
+                        for p, *ts in zip(params, grads, st['m'], st['v']) for t in (p, *ts))):
+            counts = (ctypes.c_int64 * len(params))(*[p.numel() for p in params])
+            _native.check(_native.load().xtm_adam_step(
+                len(params), _pointers(params), _pointers(grads), _pointers(st['m']),
+                _pointers(st['v']), counts, _ptr(st['t']), lr, beta1, 1 - beta1, beta2,
+                1 - beta2, eps, _stream(st['t'].device)))
+            return
         bc1 = 1.0 - torch.pow(beta1, st['t'])
         bc2 = 1.0 - torch.pow(beta2, st['t'])
-        params, grads = self.W + self.b, gW + gb
         for k, (p, g) in enumerate(zip(params, grads)):
             st['m'][k].mul_(beta1).add_(g, alpha=1 - beta1)
             st['v'][k].mul_(beta2).addcmul_(g, g, value=1 - beta2)
