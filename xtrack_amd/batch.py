@@ -113,17 +113,41 @@ class BatchTracker:
                                  'and t_sim')
         starts = np.zeros(len(particles_list) + 1, dtype=np.int64)
         starts[1:] = np.cumsum([pp._capacity for pp in particles_list])
-        hosts = [pp.to_numpy() for pp in particles_list]
         big = Particles.__new__(Particles)
         big._capacity = int(starts[-1])
         big.q0, big.mass0, big.t_sim = ref.q0, ref.mass0, ref.t_sim
         big.start_tracking_at_element = -1
+        if self._on_device(particles_list):
+            import torch
+            big._arrays = {}
+            for nn in ref._arrays:
+                parts = [pp._arrays[nn] for pp in particles_list]
+                if parts[0].dtype == torch.uint32:     # no unsigned concatenation
+                    big._arrays[nn] = torch.cat([v.view(torch.int32) for v in parts]).view(
+                        torch.uint32)
+                else:
+                    big._arrays[nn] = torch.cat(parts)
+            big._device = self.device
+            return big, starts
+        hosts = [pp.to_numpy() for pp in particles_list]
         big._arrays = {nn: np.concatenate([h[nn] for h in hosts]) for nn in hosts[0]}
         big._device = None
         big.move(_context=self.device)
         return big, starts
 
+    def _on_device(self, particles_list):
+        """Whether every particle set lives on this tracker's device: the sets
+        are then joined and parted there, without a copy through the host."""
+        return all(pp.device == self.device for pp in particles_list)
+
     def _split(self, big, starts, particles_list):
+        """Each set gets its part of the tracked set (on the device: its range
+        of the joined arrays)."""
+        if self._on_device(particles_list):
+            for nn, vv in big._arrays.items():
+                for k, pp in enumerate(particles_list):
+                    pp._arrays[nn] = vv[starts[k]:starts[k + 1]]
+            return
         host = big.to_numpy()
         for k, pp in enumerate(particles_list):
             part = {nn: np.ascontiguousarray(vv[starts[k]:starts[k + 1]])

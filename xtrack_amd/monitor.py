@@ -5,19 +5,31 @@ per-particle field, read back as ``monitor.<field>`` arrays of shape
 (n_particles, n_turns)."""
 import numpy as np
 
-from .particles import Particles, per_particle_vars
+from .particles import Particles, _device_of, _is_device_context, per_particle_vars
 
 
 def _zero_particles(n_records, device=None):
+    """n_records zero records, made where they are written: on the host, or
+    in one fill on the device (its fields are parts of one buffer)."""
     out = Particles.__new__(Particles)
-    out._capacity = int(n_records)
-    out._arrays = {nn: np.zeros(n_records, dtype=tt) for tt, nn in per_particle_vars}
+    n = out._capacity = int(n_records)
     out._device = None
+    if device is not None and _is_device_context(device):
+        import torch
+        out._device = _device_of(device)
+        buf = torch.zeros(n * sum(np.dtype(tt).itemsize for tt, _ in per_particle_vars),
+                          dtype=torch.uint8, device=out._device)
+        out._arrays, at = {}, 0
+        # the 8-byte fields come first, so every field is aligned
+        for tt, nn in per_particle_vars:
+            size = n * np.dtype(tt).itemsize
+            out._arrays[nn] = buf[at:at + size].view(getattr(torch, np.dtype(tt).name))
+            at += size
+    else:
+        out._arrays = {nn: np.zeros(n, dtype=tt) for tt, nn in per_particle_vars}
     out.q0, out.mass0, out.t_sim = 1.0, 0.0, 0.0
     out.start_at_turn = 0
     out.start_tracking_at_element = -1
-    if device is not None:
-        out.move(_context=device)
     return out
 
 
@@ -50,7 +62,7 @@ class ParticlesMonitor:
         self.data = _zero_particles(max(self.n_records, 1), device=_context)
 
     def _field(self, name):
-        vv = self.data._host_arrays()[name] if self.auto_to_numpy else self.data._arrays[name]
+        vv = self.data._host_array(name) if self.auto_to_numpy else self.data._arrays[name]
         vv = vv[:self.n_records]
         n_cols = self.stop_at_turn - self.start_at_turn
         if self.n_repetitions == 1:

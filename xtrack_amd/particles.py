@@ -274,6 +274,14 @@ class Particles:
         torch.cuda.synchronize(self._device)
         return {nn: vv.cpu().numpy() for nn, vv in self._arrays.items()}
 
+    def _host_array(self, nn):
+        """One field on the host (the array itself when it lives there)."""
+        vv = self._arrays[nn]
+        if self._device is None:
+            return vv
+        _torch().cuda.synchronize(self._device)
+        return vv.cpu().numpy()
+
     def copy(self, _context=None):
         out = Particles.__new__(Particles)
         out._capacity = self._capacity
@@ -316,8 +324,7 @@ class Particles:
     # ---- reference-style helpers -------------------------------------------
     def get_active_particle_id_range(self):
         """(min, max+1) of particle ids with state > 0 (particles.py:1340-1349)."""
-        h = self._host_arrays()
-        ids = h['particle_id'][h['state'] > 0]
+        ids = self._host_array('particle_id')[self._host_array('state') > 0]
         return int(np.min(ids)), int(np.max(ids)) + 1
 
     def reorganize(self):
@@ -371,7 +378,7 @@ class Particles:
         return self._np('zeta') / self._np('beta0')
 
     def _np(self, nn):
-        return np.asarray(self._host_arrays()[nn])
+        return np.asarray(self._host_array(nn))
 
     def __len__(self):
         return self._capacity
