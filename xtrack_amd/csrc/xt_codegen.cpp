@@ -972,11 +972,10 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
                   waves_per_eu > 0 ? waves_per_eu : 1);
     s += std::string("extern \"C\" __global__ __launch_bounds__(256) ") +
          (waves_per_eu > 0 ? occ : "") +
-         "\nvoid xtm_line_kernel(const int32_t *__restrict__ rec, const int64_t *__restrict__ entry,\n"
-         "    const double *__restrict__ prog, double line_length, xtm_particles P,\n"
-         "    int32_t num_turns, int32_t ele_start, int32_t num_ele_track,\n"
+         "\nvoid xtm_line_kernel(xtm_particles P, xtm_monitor M, const int32_t *__restrict__ rec,\n"
+         "    const int64_t *__restrict__ entry, const double *__restrict__ prog,\n"
+         "    double line_length, int32_t num_turns, int32_t ele_start, int32_t num_ele_track,\n"
          "    int32_t flag_end_turn_actions, int32_t flag_reset_s, int32_t flag_monitor,\n"
-         "    const xtm_monitor *__restrict__ Md, const xtm_particles *__restrict__ Pd,\n"
          "    uint64_t flags, int32_t num_ele_line) {\n"
          "    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;\n"
          "    const xt::TrackCtx c{flags, line_length, P.q0, P.t_sim, num_ele_line};\n"
@@ -985,7 +984,7 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
          "    xt::track_particle_units" + bt + "(P, i, alive, xt_gen::Runner{rec, entry, prog}, c,\n"
          "                             num_turns, ele_start, num_ele_track,\n"
          "                             flag_end_turn_actions, flag_reset_s, flag_monitor,\n"
-         "                             xt::MonRef{Md, Pd});\n"
+         "                             xt::kernarg());\n"
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over all particles\n"
@@ -1052,13 +1051,11 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
     s += "#if defined(__HIPCC__)\n";
     s += std::string("extern \"C\" __global__ __launch_bounds__(256) ") +
          (waves_per_eu > 0 ? occ : "") +
-         "\nvoid xtm_batch_line_kernel(const xt_gen::BatchBlock *__restrict__ blocks,\n"
+         "\nvoid xtm_batch_line_kernel(xtm_particles P, const xt_gen::BatchBlock *__restrict__ blocks,\n"
          "    const int32_t *const *__restrict__ recs, const int64_t *const *__restrict__ entries,\n"
          "    const double *const *__restrict__ progs, const int64_t *__restrict__ nele,\n"
-         "    const double *__restrict__ lengths, const xtm_particles *__restrict__ Pd,\n"
-         "    int32_t num_turns, uint64_t flags) {\n"
+         "    const double *__restrict__ lengths, int32_t num_turns, uint64_t flags) {\n"
          "    const xt_gen::BatchBlock b = xt::cptr(blocks)[blockIdx.x];\n"
-         "    const xtm_particles &P = *Pd;\n"
          "    const int64_t i = b.first + threadIdx.x;\n"
          "    const int64_t ne = xt::cptr(nele)[b.line];\n"
          "    const xt::TrackCtx c{flags, xt::cptr(lengths)[b.line], P.q0, P.t_sim, ne};\n"
@@ -1068,7 +1065,7 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "    xt::track_particle_units<false>(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
          "                             xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
          "                             num_turns, 0, (int32_t)ne, 1, 1, 0,\n"
-         "                             xt::MonRef{nullptr, Pd});\n"
+         "                             xt::MonRef{nullptr, xt::kernarg().P});\n"
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over the blocks\n"

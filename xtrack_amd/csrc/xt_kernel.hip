@@ -59,23 +59,26 @@ constexpr unsigned kLdsLine = lds_bytes(BLOCK);
 #define XTM_OCCUPANCY
 #endif
 
-/* The particles struct is read through Pd, a device copy, so that passing
-   it by reference to the out-of-line loops copies nothing into the waves'
-   scratch frames. */
+/* A tracking kernel's first parameters are the particle struct and the
+   monitor struct, by value.  Its out-of-line functions take them by pointer
+   into the kernel argument segment itself (xt::kernarg): a reference to a
+   parameter would copy it into every wave's scratch frame, and a device copy
+   written by a launch of its own cost 5 us a call and was shared by every
+   stream of a line. */
 __global__ __launch_bounds__(BLOCK) XTM_OCCUPANCY void track_kernel(
-    const int64_t *__restrict__ entry, const double *__restrict__ prog, double line_length,
-    int64_t num_ele_line, const xtm_particles *__restrict__ Pd, int32_t num_turns,
-    int32_t ele_start, int32_t num_ele_track, int32_t flag_end_turn_actions,
-    int32_t flag_reset_s, int32_t flag_monitor, const xtm_monitor *__restrict__ Md,
-    uint64_t flags, int32_t skip_chi1) {
-    const xtm_particles &P = *Pd;
+    xtm_particles P_, xtm_monitor M_, const int64_t *__restrict__ entry,
+    const double *__restrict__ prog, double line_length, int64_t num_ele_line,
+    int32_t num_turns, int32_t ele_start, int32_t num_ele_track, int32_t flag_end_turn_actions,
+    int32_t flag_reset_s, int32_t flag_monitor, uint64_t flags, int32_t skip_chi1) {
+    const xt::MonRef mon = xt::kernarg();
+    const xtm_particles &P = *mon.P;
     const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (i >= P.capacity) return;
     // after the compiled line kernel: only the particles it left (chi != 1)
     if (skip_chi1 && P.chi[i] == 1.0) return;
     xt::track_particle(P, i, entry, prog, line_length, num_ele_line, num_turns, ele_start,
-                       num_ele_track, flag_end_turn_actions, flag_reset_s, flag_monitor,
-                       xt::MonRef{Md, Pd}, flags);
+                       num_ele_track, flag_end_turn_actions, flag_reset_s, flag_monitor, mon,
+                       flags);
 }
 
 /* One block of a batch: particles [first, first + count) of line `line`. */
@@ -91,12 +94,13 @@ struct BatchBlock {
    a scalar branch as in track_kernel. */
 template <int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void batch_kernel(
-    const BatchBlock *__restrict__ blocks, const int64_t *const *__restrict__ entries,
-    const double *const *__restrict__ progs, const int64_t *__restrict__ nele,
-    const double *__restrict__ lengths, const xtm_particles *__restrict__ Pd,
-    int32_t num_turns, uint64_t flags, int32_t skip_chi1) {
+    xtm_particles P_, const BatchBlock *__restrict__ blocks,
+    const int64_t *const *__restrict__ entries, const double *const *__restrict__ progs,
+    const int64_t *__restrict__ nele, const double *__restrict__ lengths, int32_t num_turns,
+    uint64_t flags, int32_t skip_chi1) {
     const BatchBlock b = xt::cptr(blocks)[blockIdx.x];
     if ((int32_t)threadIdx.x >= b.count) return;
+    const xtm_particles *Pd = xt::kernarg().P;
     const xtm_particles &P = *Pd;
     const int64_t i = b.first + threadIdx.x;
     // after the compiled batch kernel: only the particles it left (chi != 1)
@@ -106,17 +110,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
     const xt::ProgramRunner run{xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]};
     xt::track_particle_with<false>(P, i, run, run, c, num_turns, 0, (int32_t)ne, 1, 1, 0,
                                    xt::MonRef{nullptr, Pd});
-}
-
-/* device copies of the particle struct and the monitor for the tracking
-   kernels (stream-ordered before them; kernel arguments are captured at
-   launch, so the caller's structs need not outlive the call) */
-__global__ void args_kernel(xtm_particles P, xtm_monitor M, xtm_particles *Pd,
-                            xtm_monitor *Md) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *Pd = P;
-        *Md = M;
-    }
 }
 
 /* Feature accumulators of every active particle at the start of its
@@ -197,10 +190,6 @@ struct xtm_line {
     std::vector<int64_t> entry;   // host copies (operation counting, code generation)
     std::vector<int64_t> entry_bt;
     std::vector<double> prog;
-    // device copies of the particle and monitor structs read by monitor
-    // records (written by monitor_args_kernel before a launch with a monitor)
-    xtm_particles *d_mon_p = nullptr;
-    xtm_monitor *d_mon_m = nullptr;
     // generated line code (xtm_line_specialize)
     LineCode code;
     uint32_t spec_options = 0;
@@ -224,8 +213,6 @@ struct xtm_batch {
     double *d_lengths = nullptr;
     BatchBlock *d_blocks = nullptr;
     int64_t d_blocks_cap = 0;
-    xtm_particles *d_p = nullptr;
-    xtm_monitor *d_m = nullptr;
     // generated batch code (xtm_batch_specialize)
     std::vector<int32_t *> d_recs;
     const int32_t **d_rec_ptrs = nullptr;
@@ -346,9 +333,7 @@ int32_t xtm_line_create(const int32_t *types, const int64_t *offsets, const doub
     const size_t ne = entry.empty() ? 1 : entry.size();
     if ((e = hipMalloc(&L->d_entry, ne * sizeof(int64_t))) != hipSuccess ||
         (e = hipMalloc(&L->d_entry_bt, ne * sizeof(int64_t))) != hipSuccess ||
-        (e = hipMalloc(&L->d_prog, prog.size() * sizeof(double))) != hipSuccess ||
-        (e = hipMalloc(&L->d_mon_p, sizeof(xtm_particles))) != hipSuccess ||
-        (e = hipMalloc(&L->d_mon_m, sizeof(xtm_monitor))) != hipSuccess) {
+        (e = hipMalloc(&L->d_prog, prog.size() * sizeof(double))) != hipSuccess) {
         xtm_line_destroy(L);
         return hip_fail(e, "hipMalloc");
     }
@@ -378,8 +363,6 @@ int32_t xtm_line_destroy(xtm_line *L) {
     if (L->d_entry) (void)hipFree(L->d_entry);
     if (L->d_entry_bt) (void)hipFree(L->d_entry_bt);
     if (L->d_prog) (void)hipFree(L->d_prog);
-    if (L->d_mon_p) (void)hipFree(L->d_mon_p);
-    if (L->d_mon_m) (void)hipFree(L->d_mon_m);
     L->code.release();
     L->bt.release();
     delete L;
@@ -549,12 +532,6 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
     xtm_monitor M;
     if (flag_monitor) M = *monitor;
     else std::memset(&M, 0, sizeof(M));
-    hipLaunchKernelGGL(args_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, *P, M,
-                       L->d_mon_p, L->d_mon_m);
-    e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "args_kernel launch");
-    const xtm_monitor *Md = L->d_mon_m;
-    const xtm_particles *Pd = L->d_mon_p;
     const int64_t nblocks = (P->capacity + BLOCK - 1) / BLOCK;
     if (nblocks > 0x7fffffff) return fail(XTM_ERR_ARG, "too many particles");
     const bool backtrack = (track_flags >> XTM_FLAG_BACKTRACK) & 1;
@@ -573,8 +550,8 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
         int32_t a_end = flag_end_turn_actions, a_reset = flag_reset_s_at_end_turn;
         int32_t a_mon = flag_monitor;
         uint64_t a_flags = track_flags;
-        void *args[] = {&rec, &entry, &prog, &line_length, &Pv, &a_turns, &a_start, &a_n,
-                        &a_end, &a_reset, &a_mon, &Md, &Pd, &a_flags, &a_nele};
+        void *args[] = {&Pv, &M, &rec, &entry, &prog, &line_length, &a_turns, &a_start, &a_n,
+                        &a_end, &a_reset, &a_mon, &a_flags, &a_nele};
         e = hipModuleLaunchKernel(code->kernel, (unsigned)nblocks, 1, 1, BLOCK, 1, 1, kLdsLine,
                                   (hipStream_t)stream, args, nullptr);
         if (e != hipSuccess) return hip_fail(e, "xtm_line_kernel launch");
@@ -582,11 +559,10 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
     /* the interpreter: every particle, or after the compiled code those with
        chi != 1, on the same stream */
     hipLaunchKernelGGL(track_kernel, dim3((unsigned)nblocks), dim3(BLOCK), kLdsLine,
-                       (hipStream_t)stream, backtrack ? L->d_entry_bt : L->d_entry, L->d_prog,
-                       L->line_length, (int64_t)L->num_elements, Pd,
-                       num_turns, ele_start, num_ele_track, flag_end_turn_actions,
-                       flag_reset_s_at_end_turn, flag_monitor, Md, track_flags,
-                       (int32_t)(code ? 1 : 0));
+                       (hipStream_t)stream, *P, M, backtrack ? L->d_entry_bt : L->d_entry,
+                       L->d_prog, L->line_length, (int64_t)L->num_elements, num_turns, ele_start,
+                       num_ele_track, flag_end_turn_actions, flag_reset_s_at_end_turn,
+                       flag_monitor, track_flags, (int32_t)(code ? 1 : 0));
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "track_kernel launch");
     return XTM_OK;
@@ -650,8 +626,6 @@ int32_t xtm_batch_destroy(xtm_batch *B) {
         if (B->d_nele) (void)hipFree(B->d_nele);
         if (B->d_lengths) (void)hipFree(B->d_lengths);
         if (B->d_blocks) (void)hipFree(B->d_blocks);
-        if (B->d_p) (void)hipFree(B->d_p);
-        if (B->d_m) (void)hipFree(B->d_m);
         for (int32_t *r : B->d_recs)
             if (r) (void)hipFree(r);
         if (B->d_rec_ptrs) (void)hipFree(B->d_rec_ptrs);
@@ -698,9 +672,7 @@ int32_t xtm_batch_create(xtm_line *const *lines, int32_t num_lines, xtm_batch **
     if ((e = hipMalloc(&B->d_entries, n * sizeof(int64_t *))) != hipSuccess ||
         (e = hipMalloc(&B->d_progs, n * sizeof(double *))) != hipSuccess ||
         (e = hipMalloc(&B->d_nele, n * sizeof(int64_t))) != hipSuccess ||
-        (e = hipMalloc(&B->d_lengths, n * sizeof(double))) != hipSuccess ||
-        (e = hipMalloc(&B->d_p, sizeof(xtm_particles))) != hipSuccess ||
-        (e = hipMalloc(&B->d_m, sizeof(xtm_monitor))) != hipSuccess) {
+        (e = hipMalloc(&B->d_lengths, n * sizeof(double))) != hipSuccess) {
         xtm_batch_destroy(B);
         return hip_fail(e, "hipMalloc");
     }
@@ -795,12 +767,7 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
     if (num_turns == 0 || B->blocks.empty()) return XTM_OK;
     hipError_t e = hipSetDevice(B->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
-    xtm_monitor M;
-    std::memset(&M, 0, sizeof(M));
     const hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(args_kernel, dim3(1), dim3(64), 0, s, *P, M, B->d_p, B->d_m);
-    e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "args_kernel launch");
     const dim3 grid((unsigned)B->blocks.size());
     const int64_t *const *entries = B->d_entries;
     const double *const *progs = B->d_progs;
@@ -810,10 +777,10 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
         const int32_t *const *recs = B->d_rec_ptrs;
         const int64_t *nele = B->d_nele;
         const double *lengths = B->d_lengths;
-        const xtm_particles *Pd = B->d_p;
+        xtm_particles Pv = *P;
         int32_t a_turns = num_turns;
         uint64_t a_flags = track_flags;
-        void *args[] = {&blocks, &recs, &entries, &progs, &nele, &lengths, &Pd, &a_turns,
+        void *args[] = {&Pv, &blocks, &recs, &entries, &progs, &nele, &lengths, &a_turns,
                         &a_flags};
         e = hipModuleLaunchKernel(B->kernel, grid.x, 1, 1, (unsigned)B->block_size, 1, 1,
                                   lds_bytes(B->block_size), s, args, nullptr);
@@ -823,14 +790,14 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
     const dim3 block((unsigned)B->block_size);
     const unsigned lds = lds_bytes(B->block_size);
     if (B->waves_per_eu == 5)
-        hipLaunchKernelGGL((batch_kernel<5>), grid, block, lds, s, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, B->d_p, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<5>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
+                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     else if (B->waves_per_eu == 4)
-        hipLaunchKernelGGL((batch_kernel<4>), grid, block, lds, s, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, B->d_p, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<4>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
+                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     else
-        hipLaunchKernelGGL((batch_kernel<3>), grid, block, lds, s, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, B->d_p, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<3>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
+                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "batch_kernel launch");
     return XTM_OK;

@@ -1305,14 +1305,24 @@ XT_HD_COLD void monitor_record(const xtm_monitor &M, const xtm_particles &P, int
     }
 }
 
-/* What the monitor records need: the monitor and the tracked particles'
-   struct, by pointer.  On the GPU both point to device copies, so that no
-   kernel argument has its address taken (which would copy it into every
-   wave's scratch frame). */
+/* What the out-of-line functions need: the tracked particles' struct and the
+   monitor, by pointer. */
 struct MonRef {
     const xtm_monitor *M;
     const xtm_particles *P;
 };
+
+#if defined(__HIP_DEVICE_COMPILE__)
+/* Both structs in the kernel argument segment of a kernel whose first
+   parameters are xtm_particles and xtm_monitor by value (the batch kernels:
+   xtm_particles only, and no monitor).  To be called in the kernel itself. */
+__device__ __forceinline__ MonRef kernarg() {
+    const char *a = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
+    return MonRef{(const xtm_monitor *)(a + sizeof(xtm_particles)), (const xtm_particles *)a};
+}
+#elif defined(__HIPCC__)
+__device__ MonRef kernarg();   /* host pass */
+#endif
 
 /* Feature accumulators of particle slot i at the start of a turn (see
    xtm_features), from its coordinates between two tracking launches. */
