@@ -372,8 +372,8 @@ int32_t xtm_features_record(const xtm_particles *particles, const xtm_features *
                             void *stream);
 
 /* num_turns whole turns from element 0 (end-of-turn actions on, s reset,
- * no monitor) as one-turn xtm_track_line launches, each preceded by
- * xtm_features_record: the surrogate's feature turns without a
+ * no monitor) with the record of xtm_features_record at the start of each
+ * turn, in one launch: the surrogate's feature turns without a
  * turn-by-turn record (no counterpart in the reference). */
 int32_t xtm_track_line_features(xtm_line *line, const xtm_particles *particles,
                                 int32_t num_turns, const xtm_features *features,
@@ -442,9 +442,8 @@ int32_t xtm_batch_generate_source(const xtm_batch *batch, int32_t waves_per_eu, 
 int32_t xtm_batch_track(xtm_batch *batch, const xtm_particles *particles,
                         int32_t num_turns, uint64_t track_flags, void *stream);
 
-/* xtm_batch_track as one-turn launches, each preceded by
- * xtm_features_record (as xtm_track_line_features; one normalisation for
- * all lines). */
+/* xtm_batch_track with the record of xtm_features_record at the start of
+ * each turn (as xtm_track_line_features; one normalisation for all lines). */
 int32_t xtm_batch_track_features(xtm_batch *batch, const xtm_particles *particles,
                                  int32_t num_turns, const xtm_features *features,
                                  uint64_t track_flags, void *stream);

@@ -722,11 +722,11 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         recs[l].resize(entry.size());
         for (size_t e = 0; e < entry.size(); e++) recs[l][e] = fn_of_pc[entry[e]];
     }
-
     // Segments: runs of consecutive cheap literal records (drifts,
     // apertures, thin kicks, markers) cut into chunks of at most kSegMax
-    // elements; a chunk sequence becomes one function that tracks the chunk's elements in order and
-    // returns the position of the element where the particle was lost.  The
+    // elements; a chunk sequence becomes one function that tracks the
+    // chunk's elements in order and returns the position of the element where
+    // the particle was lost.  The
     // key of a chunk's first element carries the segment number and the
     // chunk length; the loop runs the chunk with one dispatch instead of one
     // per element.  Same element calls, same order: the arithmetic is that
@@ -972,8 +972,8 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
                   waves_per_eu > 0 ? waves_per_eu : 1);
     s += std::string("extern \"C\" __global__ __launch_bounds__(256) ") +
          (waves_per_eu > 0 ? occ : "") +
-         "\nvoid xtm_line_kernel(xtm_particles P, xtm_monitor M, const int32_t *__restrict__ rec,\n"
-         "    const int64_t *__restrict__ entry, const double *__restrict__ prog,\n"
+         "\nvoid xtm_line_kernel(xtm_particles P, xtm_monitor M, xtm_features F,\n"
+         "    const int32_t *__restrict__ rec, const int64_t *__restrict__ entry, const double *__restrict__ prog,\n"
          "    double line_length, int32_t num_turns, int32_t ele_start, int32_t num_ele_track,\n"
          "    int32_t flag_end_turn_actions, int32_t flag_reset_s, int32_t flag_monitor,\n"
          "    uint64_t flags, int32_t num_ele_line) {\n"
@@ -1051,7 +1051,8 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
     s += "#if defined(__HIPCC__)\n";
     s += std::string("extern \"C\" __global__ __launch_bounds__(256) ") +
          (waves_per_eu > 0 ? occ : "") +
-         "\nvoid xtm_batch_line_kernel(xtm_particles P, const xt_gen::BatchBlock *__restrict__ blocks,\n"
+         "\nvoid xtm_batch_line_kernel(xtm_particles P, xtm_monitor M, xtm_features F,\n"
+         "    int32_t flag_monitor, const xt_gen::BatchBlock *__restrict__ blocks,\n"
          "    const int32_t *const *__restrict__ recs, const int64_t *const *__restrict__ entries,\n"
          "    const double *const *__restrict__ progs, const int64_t *__restrict__ nele,\n"
          "    const double *__restrict__ lengths, int32_t num_turns, uint64_t flags) {\n"
@@ -1064,8 +1065,8 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "                       P.chi[i] == 1.0;\n"
          "    xt::track_particle_units<false>(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
          "                             xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
-         "                             num_turns, 0, (int32_t)ne, 1, 1, 0,\n"
-         "                             xt::MonRef{nullptr, xt::kernarg().P});\n"
+         "                             num_turns, 0, (int32_t)ne, 1, 1, flag_monitor,\n"
+         "                             xt::kernarg());\n"
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over the blocks\n"

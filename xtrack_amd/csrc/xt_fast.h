@@ -391,8 +391,8 @@ XT_HD double *thread_slots(double *host_slots, int32_t *stride) {
 }
 
 /* A unit of n elements from element e with the general element code, on the
-   state in the particle's slots; with `record`, the monitor record of the
-   state before it.  n = 0: the record only.  at_element: the particle's at
+   state in the particle's slots; with `record` (flag_monitor's value), the
+   monitor or feature record of the state before it.  n = 0: the record only.  at_element: the particle's at
    the unit's first element.  A lost particle is stored, with the element of
    the unit where it was lost; returns false for it.
    Out of line: its registers and calls take no part in the common path. */
@@ -401,7 +401,7 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
                                       double *host_slots, const int64_t i, const MonRef mon,
                                       const uint64_t flags, const double line_length,
                                       const int32_t e, const int32_t n, const int64_t at_turn,
-                                      const int64_t at_element, const bool record) {
+                                      const int64_t at_element, const int32_t record) {
     const xtm_particles &P = *mon.P;
     const TrackCtx c{flags, line_length, P.q0, P.t_sim, 0};
     PState<double> p;
@@ -411,7 +411,9 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
     p.chi = 1.0;
     p.at_turn = at_turn;
     p.state = P.state[i];
-    if (record)
+    if (record == 3)
+        feature_hook(mon.F, i, p.x, p.px, p.y, p.py, at_turn);
+    else if (record)
         monitor_record(*mon.M, P, i, p.x, p.px, p.y, p.py, p.zeta, p.delta(), p.rpp(), p.rvv(),
                        p.s(), p.chi, p.at_turn, p.state, at_element, BT);
     int64_t j = 0;
@@ -484,7 +486,7 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
     };
     /* the general code on the unit; false when the particle is lost */
     auto general = [&](FState &q, const typename Runner::Key key, const int32_t e,
-                       const int32_t n, const bool record) {
+                       const int32_t n, const int32_t record) {
         slot[XS_X * stride] = p.x; slot[XS_PX * stride] = p.px;
         slot[XS_Y * stride] = p.y; slot[XS_PY * stride] = p.py;
         slot[XS_ZETA * stride] = p.zeta; slot[XS_S * stride] = p.s;
@@ -508,10 +510,10 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
         }
         typename Runner::Key key{};
         if (ele_start < ele_stop) key = run.key(ele_start);
-        if (!BT && flag_monitor == 1) {
+        if (!BT && (flag_monitor == 1 || flag_monitor == 3)) {
             store_axay();
             FState q = p;
-            if (alive) general(q, key, ele_start, 0, true);
+            if (alive) general(q, key, ele_start, 0, flag_monitor);
         }
         for (int32_t e = ele_start; e < ele_stop;) {
             int32_t n = 1;
@@ -532,7 +534,7 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
             if (__builtin_expect(wave_any(q.bad), 0)) {
                 store_axay();
                 if (q.bad) {
-                    alive = general(q, key, e, n, flag_monitor == 2);
+                    alive = general(q, key, e, n, flag_monitor == 2 ? 2 : 0);
                     e_ok = f_energy_ok(q.delta, q.rpp, q.rvv, q.inv_rvv);
                 } else if (q.axay && alive) {
                     mon.P->ax[i] = q.ax;
@@ -549,7 +551,7 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
         if (flag_monitor == 2) {
             store_axay();
             FState q = p;
-            if (alive) general(q, key, ele_stop, 0, true);
+            if (alive) general(q, key, ele_stop, 0, 2);
         }
         if (!BT && flag_end_turn_actions > 0) {
             at_turn += 1;

@@ -59,14 +59,14 @@ constexpr unsigned kLdsLine = lds_bytes(BLOCK);
 #define XTM_OCCUPANCY
 #endif
 
-/* A tracking kernel's first parameters are the particle struct and the
-   monitor struct, by value.  Its out-of-line functions take them by pointer
+/* A tracking kernel's first parameters are the particle, monitor and feature
+   structs, by value.  Its out-of-line functions take them by pointer
    into the kernel argument segment itself (xt::kernarg): a reference to a
    parameter would copy it into every wave's scratch frame, and a device copy
    written by a launch of its own cost 5 us a call and was shared by every
    stream of a line. */
 __global__ __launch_bounds__(BLOCK) XTM_OCCUPANCY void track_kernel(
-    xtm_particles P_, xtm_monitor M_, const int64_t *__restrict__ entry,
+    xtm_particles P_, xtm_monitor M_, xtm_features F_, const int64_t *__restrict__ entry,
     const double *__restrict__ prog, double line_length, int64_t num_ele_line,
     int32_t num_turns, int32_t ele_start, int32_t num_ele_track, int32_t flag_end_turn_actions,
     int32_t flag_reset_s, int32_t flag_monitor, uint64_t flags, int32_t skip_chi1) {
@@ -94,28 +94,27 @@ struct BatchBlock {
    a scalar branch as in track_kernel. */
 template <int WPE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void batch_kernel(
-    xtm_particles P_, const BatchBlock *__restrict__ blocks,
-    const int64_t *const *__restrict__ entries, const double *const *__restrict__ progs,
-    const int64_t *__restrict__ nele, const double *__restrict__ lengths, int32_t num_turns,
-    uint64_t flags, int32_t skip_chi1) {
+    xtm_particles P_, xtm_monitor M_, xtm_features F_, int32_t flag_monitor,
+    const BatchBlock *__restrict__ blocks, const int64_t *const *__restrict__ entries,
+    const double *const *__restrict__ progs, const int64_t *__restrict__ nele,
+    const double *__restrict__ lengths, int32_t num_turns, uint64_t flags, int32_t skip_chi1) {
     const BatchBlock b = xt::cptr(blocks)[blockIdx.x];
     if ((int32_t)threadIdx.x >= b.count) return;
-    const xtm_particles *Pd = xt::kernarg().P;
-    const xtm_particles &P = *Pd;
+    const xt::MonRef mon = xt::kernarg();
+    const xtm_particles &P = *mon.P;
     const int64_t i = b.first + threadIdx.x;
     // after the compiled batch kernel: only the particles it left (chi != 1)
     if (skip_chi1 && P.chi[i] == 1.0) return;
     const int64_t ne = xt::cptr(nele)[b.line];
     const xt::TrackCtx c{flags, xt::cptr(lengths)[b.line], P.q0, P.t_sim, ne};
     const xt::ProgramRunner run{xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]};
-    xt::track_particle_with<false>(P, i, run, run, c, num_turns, 0, (int32_t)ne, 1, 1, 0,
-                                   xt::MonRef{nullptr, Pd});
+    xt::track_particle_with<false>(P, i, run, run, c, num_turns, 0, (int32_t)ne, 1, 1,
+                                   flag_monitor, mon);
 }
 
 /* Feature accumulators of every active particle at the start of its
    current turn (the state the last tracking launch left), one thread per
-   particle slot: runs between one-turn tracking launches, so the tracking
-   kernels carry no trace of it. */
+   particle slot. */
 __global__ __launch_bounds__(256) void features_kernel(xtm_features F, xtm_particles P) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= P.capacity || !(P.state[i] > 0)) return;
@@ -512,8 +511,8 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
                                int32_t ele_start, int32_t num_ele_track,
                                int32_t flag_end_turn_actions,
                                int32_t flag_reset_s_at_end_turn, int32_t flag_monitor,
-                               const xtm_monitor *monitor, uint64_t track_flags,
-                               void *stream) {
+                               const xtm_monitor *monitor, const xtm_features *features,
+                               uint64_t track_flags, void *stream) {
     if (!L || !P) return fail(XTM_ERR_ARG, "xtm_track_line: null line or particles");
     if (num_turns < 0 || ele_start < 0 || num_ele_track < 0 ||
         (int64_t)ele_start + num_ele_track > L->num_elements)
@@ -532,6 +531,13 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
     xtm_monitor M;
     if (flag_monitor) M = *monitor;
     else std::memset(&M, 0, sizeof(M));
+    xtm_features F;
+    if (features) {
+        F = *features;
+        flag_monitor = 3;
+    } else {
+        std::memset(&F, 0, sizeof(F));
+    }
     const int64_t nblocks = (P->capacity + BLOCK - 1) / BLOCK;
     if (nblocks > 0x7fffffff) return fail(XTM_ERR_ARG, "too many particles");
     const bool backtrack = (track_flags >> XTM_FLAG_BACKTRACK) & 1;
@@ -550,7 +556,7 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
         int32_t a_end = flag_end_turn_actions, a_reset = flag_reset_s_at_end_turn;
         int32_t a_mon = flag_monitor;
         uint64_t a_flags = track_flags;
-        void *args[] = {&Pv, &M, &rec, &entry, &prog, &line_length, &a_turns, &a_start, &a_n,
+        void *args[] = {&Pv, &M, &F, &rec, &entry, &prog, &line_length, &a_turns, &a_start, &a_n,
                         &a_end, &a_reset, &a_mon, &a_flags, &a_nele};
         e = hipModuleLaunchKernel(code->kernel, (unsigned)nblocks, 1, 1, BLOCK, 1, 1, kLdsLine,
                                   (hipStream_t)stream, args, nullptr);
@@ -559,7 +565,7 @@ static int32_t track_line_impl(xtm_line *L, const xtm_particles *P, int32_t num_
     /* the interpreter: every particle, or after the compiled code those with
        chi != 1, on the same stream */
     hipLaunchKernelGGL(track_kernel, dim3((unsigned)nblocks), dim3(BLOCK), kLdsLine,
-                       (hipStream_t)stream, *P, M, backtrack ? L->d_entry_bt : L->d_entry,
+                       (hipStream_t)stream, *P, M, F, backtrack ? L->d_entry_bt : L->d_entry,
                        L->d_prog, L->line_length, (int64_t)L->num_elements, num_turns, ele_start,
                        num_ele_track, flag_end_turn_actions, flag_reset_s_at_end_turn,
                        flag_monitor, track_flags, (int32_t)(code ? 1 : 0));
@@ -573,7 +579,7 @@ int32_t xtm_track_line(xtm_line *L, const xtm_particles *P, int32_t num_turns,
                        int32_t flag_reset_s_at_end_turn, int32_t flag_monitor,
                        const xtm_monitor *monitor, uint64_t track_flags, void *stream) {
     return track_line_impl(L, P, num_turns, ele_start, num_ele_track, flag_end_turn_actions,
-                           flag_reset_s_at_end_turn, flag_monitor, monitor, track_flags,
+                           flag_reset_s_at_end_turn, flag_monitor, monitor, nullptr, track_flags,
                            stream);
 }
 
@@ -598,16 +604,13 @@ int32_t xtm_track_line_features(xtm_line *L, const xtm_particles *P, int32_t num
         return fail(XTM_ERR_ARG, "xtm_track_line_features: null argument");
     if ((track_flags >> XTM_FLAG_BACKTRACK) & 1)
         return fail(XTM_ERR_UNSUPPORTED, "xtm_track_line_features: tracks forward only");
-    for (int32_t t = 0; t < num_turns; t++) {
-        int32_t st = xtm_features_record(P, features, stream);
-        if (st == XTM_OK)
-            st = track_line_impl(L, P, 1, 0, (int32_t)L->num_elements, 1, 1, 0, nullptr,
-                                 track_flags, stream);
-        if (st != XTM_OK) return st;
-    }
-    return XTM_OK;
+    if (num_turns <= 0) return XTM_OK;
+    if (!features_ok(features, P->capacity))
+        return fail(XTM_ERR_ARG, "xtm_features_record: accumulators missing or of the wrong "
+                                 "capacity");
+    return track_line_impl(L, P, num_turns, 0, (int32_t)L->num_elements, 1, 1, 0, nullptr,
+                           features, track_flags, stream);
 }
-
 
 int32_t xtm_line_count_ops(const xtm_line *L, const double *coords, double p0c,
                            double mass0, double q0, double *out) {
@@ -752,7 +755,8 @@ int32_t xtm_batch_copy_blocks(const xtm_batch *B, int64_t *out) {
 }
 
 static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t num_turns,
-                                uint64_t track_flags, void *stream) {
+                                const xtm_features *features, uint64_t track_flags,
+                                void *stream) {
     if (!B || !P) return fail(XTM_ERR_ARG, "xtm_batch_track: null batch or particles");
     if (B->device < 0) return fail(XTM_ERR_ARG, "xtm_batch_track: batch was created without a device");
     if (B->line_start.empty()) return fail(XTM_ERR_ARG, "xtm_batch_track: no layout set");
@@ -768,6 +772,16 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
     hipError_t e = hipSetDevice(B->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     const hipStream_t s = (hipStream_t)stream;
+    xtm_monitor M;
+    std::memset(&M, 0, sizeof(M));
+    xtm_features F;
+    int32_t a_mon = 0;
+    if (features) {
+        F = *features;
+        a_mon = 3;
+    } else {
+        std::memset(&F, 0, sizeof(F));
+    }
     const dim3 grid((unsigned)B->blocks.size());
     const int64_t *const *entries = B->d_entries;
     const double *const *progs = B->d_progs;
@@ -780,7 +794,7 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
         xtm_particles Pv = *P;
         int32_t a_turns = num_turns;
         uint64_t a_flags = track_flags;
-        void *args[] = {&Pv, &blocks, &recs, &entries, &progs, &nele, &lengths, &a_turns,
+        void *args[] = {&Pv, &M, &F, &a_mon, &blocks, &recs, &entries, &progs, &nele, &lengths, &a_turns,
                         &a_flags};
         e = hipModuleLaunchKernel(B->kernel, grid.x, 1, 1, (unsigned)B->block_size, 1, 1,
                                   lds_bytes(B->block_size), s, args, nullptr);
@@ -790,14 +804,14 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
     const dim3 block((unsigned)B->block_size);
     const unsigned lds = lds_bytes(B->block_size);
     if (B->waves_per_eu == 5)
-        hipLaunchKernelGGL((batch_kernel<5>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<5>), grid, block, lds, s, *P, M, F, a_mon, B->d_blocks,
+                           entries, progs, B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     else if (B->waves_per_eu == 4)
-        hipLaunchKernelGGL((batch_kernel<4>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<4>), grid, block, lds, s, *P, M, F, a_mon, B->d_blocks,
+                           entries, progs, B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     else
-        hipLaunchKernelGGL((batch_kernel<3>), grid, block, lds, s, *P, B->d_blocks, entries, progs,
-                           B->d_nele, B->d_lengths, num_turns, track_flags, skip);
+        hipLaunchKernelGGL((batch_kernel<3>), grid, block, lds, s, *P, M, F, a_mon, B->d_blocks,
+                           entries, progs, B->d_nele, B->d_lengths, num_turns, track_flags, skip);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "batch_kernel launch");
     return XTM_OK;
@@ -805,7 +819,7 @@ static int32_t batch_track_impl(xtm_batch *B, const xtm_particles *P, int32_t nu
 
 int32_t xtm_batch_track(xtm_batch *B, const xtm_particles *P, int32_t num_turns,
                         uint64_t track_flags, void *stream) {
-    return batch_track_impl(B, P, num_turns, track_flags, stream);
+    return batch_track_impl(B, P, num_turns, nullptr, track_flags, stream);
 }
 
 int32_t xtm_batch_track_features(xtm_batch *B, const xtm_particles *P, int32_t num_turns,
@@ -813,9 +827,13 @@ int32_t xtm_batch_track_features(xtm_batch *B, const xtm_particles *P, int32_t n
                                  void *stream) {
     if (!B || !P || !features)
         return fail(XTM_ERR_ARG, "xtm_batch_track_features: null argument");
+    if (num_turns > 0 && !B->line_start.empty() && P->capacity == B->line_start.back() &&
+        !B->blocks.empty() && features_ok(features, P->capacity))
+        return batch_track_impl(B, P, num_turns, features, track_flags, stream);
+    // slots outside the layout are recorded, too, but not tracked
     for (int32_t t = 0; t < num_turns; t++) {
         int32_t st = xtm_features_record(P, features, stream);
-        if (st == XTM_OK) st = batch_track_impl(B, P, 1, track_flags, stream);
+        if (st == XTM_OK) st = batch_track_impl(B, P, 1, nullptr, track_flags, stream);
         if (st != XTM_OK) return st;
     }
     return XTM_OK;

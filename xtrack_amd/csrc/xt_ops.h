@@ -1310,15 +1310,18 @@ XT_HD_COLD void monitor_record(const xtm_monitor &M, const xtm_particles &P, int
 struct MonRef {
     const xtm_monitor *M;
     const xtm_particles *P;
+    const xtm_features *F;   /* flag_monitor 3: feature accumulators */
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
-/* Both structs in the kernel argument segment of a kernel whose first
-   parameters are xtm_particles and xtm_monitor by value (the batch kernels:
-   xtm_particles only, and no monitor).  To be called in the kernel itself. */
+/* The structs in the kernel argument segment of a tracking kernel, whose first
+   parameters are xtm_particles, xtm_monitor and xtm_features by value.  To be
+   called in the kernel itself. */
 __device__ __forceinline__ MonRef kernarg() {
     const char *a = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
-    return MonRef{(const xtm_monitor *)(a + sizeof(xtm_particles)), (const xtm_particles *)a};
+    const char *m = a + sizeof(xtm_particles);
+    return MonRef{(const xtm_monitor *)m, (const xtm_particles *)a,
+                  (const xtm_features *)(m + sizeof(xtm_monitor))};
 }
 #elif defined(__HIPCC__)
 __device__ MonRef kernarg();   /* host pass */
@@ -1378,6 +1381,14 @@ XT_HD void feature_record(const xtm_features &F, const int64_t i, const double x
     n = n + 1.0;
 }
 
+/* the record between a tracking kernel's turns, out of line: a turn of the
+   element loop carries none of its registers */
+XT_HD_COLD void feature_hook(const xtm_features *F, const int64_t i, const double x,
+                             const double px, const double y, const double py,
+                             const int64_t at_turn) {
+    feature_record(*F, i, x, px, y, py, at_turn);
+}
+
 #define XT_MONITOR_RECORD(AT_ELEMENT)                                                     \
     monitor_record(*mon.M, *mon.P, i, p.x, p.px, p.y, p.py, p.zeta, p.delta(), p.rpp(),       \
                    p.rvv(), p.s(), p.chi, p.at_turn, p.state, (AT_ELEMENT), BT)
@@ -1435,6 +1446,8 @@ XT_HD void track_particle_loop(const xtm_particles &P, int64_t i, const Runner &
         int64_t base = P.at_element[i] - ele_start;
         for (int32_t iturn = 0; iturn < num_turns; iturn++) {
             if (flag_monitor == 1) XT_MONITOR_RECORD(base + ele_start);
+            if (flag_monitor == 3)
+                feature_hook(mon.F, i, p.x, p.px, p.y, p.py, p.at_turn);
             /* the next element's key (record index / program offset) is
                loaded one element ahead, so its scalar load overlaps the
                current element's arithmetic */

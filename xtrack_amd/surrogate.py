@@ -383,7 +383,7 @@ def track_features(line_or_batch, particles, num_turns, inv_w4, co, sx, sy, star
                    acc=None, window=None):
     """Track `particles` (a device particle set) for num_turns whole turns
     with the feature accumulators updated on the device at the start of every
-    turn, between one-turn tracking launches (xtm_track_line_features /
+    turn, in the tracking launch (xtm_track_line_features /
     xtm_batch_track_features);
     returns the accumulators, a (XTM_FEAT_N, capacity) float64 tensor on the
     device, row k = accumulator k of every particle slot.
