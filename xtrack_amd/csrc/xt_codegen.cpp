@@ -15,6 +15,7 @@
 #include <cinttypes>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -211,7 +212,11 @@ struct FastGen {
     bool direct = false;   // holds an op that only the general code has
     bool axay = false;     // sets ax and ay
 
-    FastGen(const std::vector<double> &p, bool l) : prog(p), loads(l) {}
+    // loaded constants that every record of the structure shares: literals
+    const std::vector<char> *shared;
+
+    FastGen(const std::vector<double> &p, bool l, const std::vector<char> *s = nullptr)
+        : prog(p), loads(l), shared(s) {}
 
     static constexpr double kInf = 1e300;
     static constexpr double kRange = 0x1p100;   // products of a few stay finite
@@ -221,7 +226,8 @@ struct FastGen {
     bool signs = false;
 
     std::string c(int64_t i) const {
-        if (loads) return "rp[" + std::to_string(i - base) + "]";
+        if (loads && !(shared && i - base < (int64_t)shared->size() && (*shared)[i - base]))
+            return "rp[" + std::to_string(i - base) + "]";
         return lit(prog[i]);
     }
     std::string cs(int64_t i, int n) const {
@@ -686,8 +692,9 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         const auto &info = lit_info[*r.second];
         cs.small.push_back(!info.first && info.second <= kSmallCost);
     }
-    // the other records: structure functions
+    // the other records: structure functions, and the records of each
     std::map<std::string, int32_t> fn_of_struct;
+    std::map<int32_t, std::vector<std::pair<size_t, int64_t>>> records_of;
     recs.assign(nl, {});
     for (size_t l = 0; l < nl; l++) {
         std::map<int64_t, int32_t> fn_of_pc;
@@ -712,6 +719,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                 cs.small.push_back(0);
             }
             fn_of_pc.emplace(pu.first, ins.first->second);
+            records_of[ins.first->second].emplace_back(l, pu.first);
         }
         if ((int64_t)cs.body.size() > XT_CODEGEN_MAX_RECORDS) {
             err = "the code needs more than " + std::to_string(XT_CODEGEN_MAX_RECORDS) +
@@ -722,6 +730,32 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         recs[l].resize(entry.size());
         for (size_t e = 0; e < entry.size(); e++) recs[l][e] = fn_of_pc[entry[e]];
     }
+    // Constants that all records of a structure share become literals of its
+    // unit code: bends with their own field errors load 5 words instead of
+    // 150, and a wave alone on its SIMD waits for the scalar loads of each
+    // element.  Error ring, 64,000 particles, one turn: 11.7 -> 8.8 ms.
+    for (auto &kv : records_of) {
+        const size_t l0 = kv.second[0].first;
+        const int64_t pc0 = kv.second[0].second;
+        std::vector<char> shared;
+        const std::string &text = cs.fast[kv.first];
+        for (size_t q = text.find("rp["); q != std::string::npos; q = text.find("rp[", q + 3)) {
+            const int64_t k = std::strtoll(text.c_str() + q + 3, nullptr, 10);
+            if (k >= (int64_t)shared.size()) shared.resize(k + 1, 0);
+            shared[k] = 1;
+        }
+        for (size_t k = 0; k < shared.size(); k++)
+            for (auto &rc : kv.second)
+                shared[k] = shared[k] && wbits((*progs[rc.first])[rc.second + k]) ==
+                                             wbits((*progs[l0])[pc0 + k]);
+        FastGen f(*progs[l0], true, &shared);
+        if (!f.record(pc0)) {
+            err = "cannot generate unit code at program offset " + std::to_string(pc0);
+            return XTM_ERR_ARG;
+        }
+        cs.fast[kv.first] = f.body();
+    }
+
     // Segments: runs of consecutive cheap literal records (drifts,
     // apertures, thin kicks, markers) cut into chunks of at most kSegMax
     // elements; a chunk sequence becomes one function that tracks the
