@@ -171,8 +171,8 @@ struct Gen {
             case OP_EDGE_CLEAR_AXAY: line("xt::op_edge_clear_axay(m);"); break;
             case OP_EDGE_LINEAR: line("xt::op_edge_linear(p" + cs(a, 2) + ");"); break;
             case OP_RF_KICK:
-                line("xt::op_rf_kick(p, m, " + at +
-                     ", c.line_length, c.q0, c.t_sim, c.kill_energy());");
+                line("xt::op_rf_kick(p, m" + cs(a, 5) + ", xt::wbits(" + c(a + 5) +
+                     "), c.line_length, c.q0, c.t_sim, c.kill_energy());");
                 break;
             case OP_LIMIT_RECT:
                 line("xt::op_limit_rect(p" + cs(a, 4) + ", c.ignore_local());");

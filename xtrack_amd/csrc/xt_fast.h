@@ -392,9 +392,11 @@ XT_HD double *thread_slots(double *host_slots, int32_t *stride) {
 
 /* A unit of n elements from element e with the general element code, on the
    state in the particle's slots; with `record` (flag_monitor's value), the
-   monitor or feature record of the state before it.  n = 0: the record only.  at_element: the particle's at
-   the unit's first element.  A lost particle is stored, with the element of
-   the unit where it was lost; returns false for it.
+   monitor or feature record of the state before it.  n = 0: the record only.
+   at_element: the particle's at the unit's first element.  A lost particle is
+   stored, with the element of the unit where it was lost; returns false for it.
+   The number in P.state is loaded for the records alone: the elements only
+   set it, and a function call would wait for the load.
    Out of line: its registers and calls take no part in the common path. */
 template <bool BT, class Runner>
 XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key key,
@@ -410,7 +412,7 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
     p.zeta = p.get(XS_ZETA);
     p.chi = 1.0;
     p.at_turn = at_turn;
-    p.state = P.state[i];
+    p.state = record ? P.state[i] : 1;
     if (record == 3)
         feature_hook(mon.F, i, p.x, p.px, p.y, p.py, at_turn);
     else if (record)

@@ -768,14 +768,9 @@ XT_HD void update_ptau(PState<R> &p, R new_ptau, const PRef &m) {
 template <class R>
 XT_HD_COLD R rf_kick_ptau(const R zeta, const R ptau_in, const R beta0, const R charge_ratio,
                           const R chi, const R p0c, const int64_t at_turn,
-                          const double *__restrict__ a, double line_length, double q0,
-                          double t_sim) {
-    const double voltage = a[0];
-    const double frequency0 = a[1];
-    const double harmonic = a[2];
-    const double lag = a[3];
-    const double phase = a[4];
-    const int64_t absolute_time = wbits(a[5]);
+                          const double voltage, const double frequency0, const double harmonic,
+                          const double lag, const double phase, const int64_t absolute_time,
+                          double line_length, double q0, double t_sim) {
     R phase0 = R(0.0);
     R frequency = R(frequency0);
     if (harmonic != 0) {
@@ -963,15 +958,17 @@ XT_HD void op_edge_linear(PState<R> &p, const double r21, const double r43) {
     p.py = p.py + chi * r43 * y;
 }
 
-/* a = the six RF arguments */
-template <class R, class PP>
-XT_HD void op_rf_kick(PState<R> &p, const PRef &m, const PP a, const double line_length,
-                      const double q0, const double t_sim, const bool kill_cavity) {
+template <class R>
+XT_HD void op_rf_kick(PState<R> &p, const PRef &m, const double voltage, const double frequency,
+                      const double harmonic, const double lag, const double phase,
+                      const int64_t absolute_time, const double line_length, const double q0,
+                      const double t_sim, const bool kill_cavity) {
     if (kill_cavity) return;
     update_ptau(p,
                 rf_kick_ptau(p.zeta, R(m.P->ptau[m.i]), R(m.P->beta0[m.i]),
                              R(m.P->charge_ratio[m.i]), p.chi, R(m.P->p0c[m.i]), p.at_turn,
-                             (const double *)a, line_length, q0, t_sim),
+                             voltage, frequency, harmonic, lag, phase, absolute_time,
+                             line_length, q0, t_sim),
                 m);
 }
 
@@ -1181,7 +1178,8 @@ XT_HD void run_element(PState<R> &p, const PRef &m, const CProg prog, int64_t pc
             pc += 3;
             break;
         case OP_RF_KICK:
-            op_rf_kick(p, m, a, c.line_length, c.q0, c.t_sim, c.kill_energy());
+            op_rf_kick(p, m, a[0], a[1], a[2], a[3], a[4], wbits(a[5]), c.line_length, c.q0,
+                       c.t_sim, c.kill_energy());
             pc += 7;
             break;
         case OP_LIMIT_RECT:
