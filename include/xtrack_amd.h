@@ -306,8 +306,10 @@ int64_t xtm_line_num_records(const xtm_line *line);
  * generation and compilation at build_tracker time (xtrack/tracker.py:
  * 544-751, compiled by xobjects): here the generated source has one
  * straight-line function per distinct element record with the record's
- * constants as literals, calling the same element maps as the program
- * interpreter, and is compiled with hiprtc for gfx950.  waves_per_eu: the
+ * constants as literals, with the results of the program interpreter's
+ * element maps, and is compiled with hiprtc for gfx950.  The code for
+ * XTM_FLAG_BACKTRACK is compiled by the first such xtm_track_line call (while
+ * the stream is captured that call runs on the interpreter).  waves_per_eu: the
  * kernel's occupancy target (0: the library default).  Returns
  * XTM_ERR_UNSUPPORTED, leaving the interpreter in use, when the line has
  * more distinct records than code is generated for; XTM_ERR_HIP when
@@ -395,8 +397,8 @@ int32_t xtm_line_count_ops(const xtm_line *line, const double *coords, double p0
  * line per `Line.track` call (xtrack/tracker.py:1372, one `track_line`
  * launch per call); each variant's particles get exactly what that call
  * gives them for full turns from element 0 (end-of-turn actions on, s
- * reset at the end of each turn, no monitor).  The lines run on the
- * element-program interpreter. */
+ * reset at the end of each turn, no monitor).  The lines run on compiled
+ * code after xtm_batch_specialize, else on the element-program interpreter. */
 typedef struct xtm_batch xtm_batch;
 
 /* A batch over `num_lines` line handles (all on one device, or all

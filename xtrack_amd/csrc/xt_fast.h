@@ -13,6 +13,18 @@
  * so the repeats are rare, and results are those of the general code bit
  * for bit.
  *
+ * What bounds it.  With many waves (a million particles) the issue of vector
+ * instructions, over 95 % of the cycles, on the thick ring 92 % of them polar
+ * drifts: a polar drift takes 72 FP64 instructions and one quarter-rate
+ * estimate here against 98, four and the range tests before, and the energy
+ * fields come from registers.  Thick ring, 28,338 elements, 1,000,000
+ * particles, one turn: 128.1 -> 92.4 ms (2.99 M vector instructions a wave
+ * against 3.90 M; 3, 4 and 5 waves per SIMD 92.6, 92.8, 92.0 ms).  With one
+ * wave per SIMD or fewer the chain of dependent operations: 64 particles
+ * 13.4 -> 7.2 ms; thin six-cell lattice, 10,000 particles, 100 turns
+ * 5.56 -> 1.00 ms, where the branches, calls and LDS reads of the general
+ * code were most of the time.
+ *
  * Exact quotients.  Every quotient, reciprocal and square root here is the
  * correctly rounded one.
  *

@@ -47,9 +47,10 @@ constexpr unsigned kLdsLine = lds_bytes(BLOCK);
 #define XTM_WAVES_PER_EU 4
 #endif
 /* Occupancy target of compiled line code (xtm_line_specialize with
-   waves_per_eu = 0).  Its per-record straight-line code needs fewer
-   registers per op than the interpreter's dispatch loop; on MI355X five
-   waves per SIMD measured fastest on the thick ring (3, 4, 6 slower). */
+   waves_per_eu = 0).  Its straight-line units fit 96 VGPRs, and the vector
+   issue that bounds them is full from three waves on: 3, 4 and 5 waves per
+   SIMD take 92.6, 92.8 and 92.0 ms for a turn of 1,000,000 particles on the
+   thick ring. */
 #ifndef XTM_COMPILED_WAVES_PER_EU
 #define XTM_COMPILED_WAVES_PER_EU 5
 #endif
