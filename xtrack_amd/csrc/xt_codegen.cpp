@@ -632,6 +632,11 @@ struct CodeSet {
     std::vector<std::string> fast_segs;        // their unit code
 };
 
+// key of a function: its general and its unit code
+std::string both(const std::string &general, const std::string &unit) {
+    return general + '\n' + unit;
+}
+
 int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                    const std::vector<const std::vector<double> *> &progs, bool keyed_pc,
                    CodeSet &cs, std::vector<std::vector<int32_t>> &recs, std::string &err) {
@@ -645,13 +650,20 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     }
     const bool all_literal = !keyed_pc && nl == 1 && n_distinct <= kLiteralAll;
     cs.keyed_pc = !all_literal;
-    // literal text of every record (program addresses relative to the
-    // record unless every record of a single line is literal)
-    std::map<std::string, int64_t> lit_uses;
-    std::vector<std::map<int64_t, std::string>> lit_text(nl);
-    std::map<std::string, std::pair<bool, int>> lit_info;   // heavy, cost
-    std::map<std::string, std::string> fast_of_lit, struct_of_lit;
-    std::map<std::string, int64_t> lits_of_struct;         // distinct literal texts
+    // literal code of every record (program addresses relative to the
+    // record unless every record of a single line is literal).  Records share
+    // a function when their general and their unit code are both the same:
+    // the general code of OP_YOSHIDA6_BEND reads its constants from the
+    // record, so bends of different lengths can agree in it, while the unit
+    // code holds every constant as a literal.
+    struct Literal {
+        std::string general, unit, structure;
+        int64_t uses = 0;
+        bool small = false;
+    };
+    std::map<std::string, Literal> lits;                   // by both texts
+    std::vector<std::map<int64_t, const std::string *>> lit_key(nl);
+    std::map<std::string, int64_t> lits_of_struct;         // distinct literal codes
     for (size_t l = 0; l < nl; l++)
         for (auto &pu : uses[l]) {
             Gen g(*progs[l], pu.first, false, !all_literal);
@@ -663,34 +675,40 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                       " at program offset " + std::to_string(pu.first);
                 return XTM_ERR_ARG;
             }
-            lit_uses[g.out] += pu.second;
-            lit_info[g.out] = {g.heavy, g.cost};
-            lit_text[l][pu.first] = g.out;
-            fast_of_lit.emplace(g.out, f.body());
-            // a structure is its general and its unit code: records of one
-            // op sequence differ in the latter where a form depends on the
-            // ranges of their constants
-            const std::string st = gs.out + fs.body();
-            if (struct_of_lit.emplace(g.out, st).second) lits_of_struct[st]++;
+            const std::string unit = f.body();
+            auto ins = lits.emplace(both(g.out, unit), Literal());
+            Literal &v = ins.first->second;
+            if (ins.second) {
+                v.general = g.out;
+                v.unit = unit;
+                // a structure is its general and its unit code: records of
+                // one op sequence differ in the latter where a form depends
+                // on the ranges of their constants
+                v.structure = both(gs.out, fs.body());
+                v.small = !g.heavy && g.cost <= kSmallCost;
+                lits_of_struct[v.structure]++;
+            }
+            v.uses += pu.second;
+            lit_key[l][pu.first] = &ins.first->first;
         }
     // A structure that the set holds with many different constants (the
     // bends of ring variants with different cell counts) gets one structure
     // function rather than a literal copy per constant set.
     std::vector<std::pair<int64_t, const std::string *>> ranked;
-    for (auto &kv : lit_uses)
+    for (auto &kv : lits)
         if (all_literal ||
-            (kv.second >= 2 && lits_of_struct[struct_of_lit[kv.first]] <= kLiteralPerStruct))
-            ranked.emplace_back(kv.second, &kv.first);
+            (kv.second.uses >= 2 && lits_of_struct[kv.second.structure] <= kLiteralPerStruct))
+            ranked.emplace_back(kv.second.uses, &kv.first);
     std::stable_sort(ranked.begin(), ranked.end(),
                      [](const auto &x, const auto &y) { return x.first > y.first; });
     if ((int64_t)ranked.size() > kLiteralMax) ranked.resize(kLiteralMax);
     std::map<std::string, int32_t> fn_of_lit;
     for (auto &r : ranked) {
+        const Literal &v = lits[*r.second];
         fn_of_lit.emplace(*r.second, (int32_t)cs.body.size());
-        cs.body.push_back(*r.second);
-        cs.fast.push_back(fast_of_lit[*r.second]);
-        const auto &info = lit_info[*r.second];
-        cs.small.push_back(!info.first && info.second <= kSmallCost);
+        cs.body.push_back(v.general);
+        cs.fast.push_back(v.unit);
+        cs.small.push_back(v.small);
     }
     // the other records: structure functions, and the records of each
     std::map<std::string, int32_t> fn_of_struct;
@@ -699,7 +717,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     for (size_t l = 0; l < nl; l++) {
         std::map<int64_t, int32_t> fn_of_pc;
         for (auto &pu : uses[l]) {
-            auto it = fn_of_lit.find(lit_text[l][pu.first]);
+            auto it = fn_of_lit.find(*lit_key[l][pu.first]);
             if (it != fn_of_lit.end()) {
                 fn_of_pc.emplace(pu.first, it->second);
                 continue;
@@ -712,7 +730,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                 return XTM_ERR_ARG;
             }
             const std::string fast = f.body();
-            auto ins = fn_of_struct.emplace(g.out + fast, (int32_t)cs.body.size());
+            auto ins = fn_of_struct.emplace(both(g.out, fast), (int32_t)cs.body.size());
             if (ins.second) {
                 cs.body.push_back(g.out);
                 cs.fast.push_back(fast);
