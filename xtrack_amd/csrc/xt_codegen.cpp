@@ -211,6 +211,7 @@ struct FastGen {
     std::string out;
     bool direct = false;   // holds an op that only the general code has
     bool axay = false;     // sets ax and ay
+    int gain = 0;          // of the unit over the general code in the loop (weight())
 
     // loaded constants that every record of the structure shares: literals
     const std::vector<char> *shared;
@@ -435,6 +436,7 @@ struct FastGen {
         }
         guard_range();
         guard_signs();
+        gain += 200;
         line(std::string("xt::f_quad<") + (k1 > 0 ? "true" : "false") + ">(p, " + c(a) + ", " +
              c(a + 2) + ");");
         const double x = 2 * bx + 4 * std::fabs(L) * bpx, y = 2 * by + 4 * std::fabs(L) * bpy;
@@ -443,6 +445,19 @@ struct FastGen {
         bx = x;
         by = y;
         if (loads) bx = by = bpx = bpy = kInf;
+    }
+
+    /* What the record gains in the loop over units against the loop over
+       general code (build_code_set: units), in units of a tenth of what a
+       drift, a thin kick or an aperture gains in a segment (0.1 us on 64
+       particles, 0.25 us on 300,000).  Measured per element: a thick
+       quadrupole 2 us, a polar drift 0.2 us, single thin elements half of
+       those in segments; a record without unit code loses 0.7 to 2.4 us to its
+       out-of-line call, less the more of its time is in functions that are out
+       of line anyway; exact bend maps gain 0.7 us there. */
+    int weight(bool small) const {
+        if (direct) return gain;
+        return (small ? 10 : 5) + gain;
     }
 
     static int drifts(int64_t op) {
@@ -464,6 +479,7 @@ struct FastGen {
         base = pc;
         std::vector<int64_t> ops;
         int n_drifts = 0;
+        bool exact_bend = false;
         for (;;) {
             if (!in_range(pc, 1) || ops.size() > 100000) return false;
             const int64_t op = wbits(prog[pc]);
@@ -472,8 +488,10 @@ struct FastGen {
             if (!in_range(pc + 1, kNargs[op])) return false;
             ops.push_back(pc);
             n_drifts += drifts(op);
+            exact_bend |= op == OP_BEND_CURVED || op == OP_BEND_STRAIGHT;
             pc += 1 + kNargs[op];
         }
+        const int all_drifts = n_drifts;
         // ops [first, first + period * count) repeat the first period
         size_t first = 0, period = 0, count = 0;
         if (n_drifts > kMaxDrifts) {
@@ -490,11 +508,14 @@ struct FastGen {
                 }
             for (size_t k = first; count && k < first + period * (count - 1); k++)
                 n_drifts -= drifts(wbits(prog[ops[k]]));
-            if (n_drifts > kMaxDrifts) {
-                direct = true;
-                return true;
-            }
+            if (n_drifts > kMaxDrifts) direct = true;
         }
+        // the rest of the record may still find that it is direct
+        auto finish = [&]() {
+            gain += direct ? (exact_bend ? 50 : -200 - 10 * all_drifts) : 20 * all_drifts;
+            return true;
+        };
+        if (direct) return finish();
         for (size_t k = 0; k < ops.size(); k++) {
             if (count && k == first) {
                 flush_limits();
@@ -504,14 +525,14 @@ struct FastGen {
                 line("for (int step = 0; step < " + std::to_string(count) + "; step++) {");
             }
             if (!emit(ops[k])) return false;
-            if (direct) return true;
+            if (direct) return finish();
             if (count && k == first + period - 1) {
                 flush_limits();
                 line("}");
                 k = first + period * count - 1;
             }
         }
-        return true;
+        return finish();
     }
 
     bool emit(int64_t pc) {
@@ -597,6 +618,12 @@ struct FastGen {
             line("xt::f_limit_ellipse(p" + cs(a, 3) + ");");
             break;
         case OP_GLOBAL_APER: convex(glob, "xt::f_global_aper(p);"); break;
+        case OP_S_SHIFT:
+            line("xt::f_s_shift(p, " + c(a) + ");");
+            bpx = bpy = 0.25;
+            bx += loads ? kInf : 2 * std::fabs(prog[a]);
+            by += loads ? kInf : 2 * std::fabs(prog[a]);
+            break;
         default:
             // RF, frame rotations, exact bends: the general code
             direct = true;
@@ -627,6 +654,7 @@ struct CodeSet {
     std::vector<std::string> body;             // function bodies (general code)
     std::vector<std::string> fast;             // their unit code
     std::vector<char> small;                   // cheap literal records
+    bool units = true;                         // the loop over units (xt_fast.h)
     bool keyed_pc = false;                     // keys carry the program offset
     std::vector<std::vector<int32_t>> segs;    // segment function bodies
     std::vector<std::string> fast_segs;        // their unit code
@@ -660,10 +688,12 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         std::string general, unit, structure;
         int64_t uses = 0;
         bool small = false;
+        int weight = 0;
     };
     std::map<std::string, Literal> lits;                   // by both texts
     std::vector<std::map<int64_t, const std::string *>> lit_key(nl);
     std::map<std::string, int64_t> lits_of_struct;         // distinct literal codes
+    int64_t gain = 0;
     for (size_t l = 0; l < nl; l++)
         for (auto &pu : uses[l]) {
             Gen g(*progs[l], pu.first, false, !all_literal);
@@ -686,11 +716,22 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                 // on the ranges of their constants
                 v.structure = both(gs.out, fs.body());
                 v.small = !g.heavy && g.cost <= kSmallCost;
+                v.weight = f.weight(v.small);
                 lits_of_struct[v.structure]++;
             }
             v.uses += pu.second;
+            gain += v.weight * pu.second;
             lit_key[l][pu.first] = &ins.first->first;
         }
+    // The loop over units suits a set whose elements gain more by their unit
+    // code than those without one lose by their out-of-line calls; the other
+    // sets run general code in the element loop.  On 64 / 300,000 particles,
+    // us a turn, general code against units: 100 quadrupoles that are off
+    // 111 / 310 against 186 / 493, 100 cavities 135 / 398 against 219 / 631,
+    // 100 RF multipoles 1016 / 3702 against 1165 / 5059; 60 quadrupoles that
+    // are off among 60 that are on 278 / 895 against 215 / 710, 108 thin kicks
+    // with 12 rotated ones 61 / 194 against 47 / 151.
+    cs.units = gain >= 0;
     // A structure that the set holds with many different constants (the
     // bends of ring variants with different cell counts) gets one structure
     // function rather than a literal copy per constant set.
@@ -901,6 +942,8 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
 /* The functions, segments and element runner of a code set, in namespace
    xt_gen. */
 std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what) {
+    const size_t n_fast = cs.units ? cs.fast.size() : 0;
+    const size_t n_fast_segs = cs.units ? cs.fast_segs.size() : 0;
     std::string s;
     s += std::string("// generated ") + what + ": element records as straight-line calls\n";
     if (options & XTM_SPEC_FAST_ARITH) s += "#define XTM_ARITH_FAST 1\n";
@@ -917,10 +960,10 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
         s += cs.body[r];
         s += "}\n\n";
     }
-    for (size_t r = 0; r < cs.fast.size(); r++)
+    for (size_t r = 0; r < n_fast; r++)
         s += "XT_GEN_FN void fast_" + std::to_string(r) +
              "(xt::FState &p, xt::CProg rp) {\n    (void)p; (void)rp;\n" + cs.fast[r] + "}\n\n";
-    for (size_t q = 0; q < cs.fast_segs.size(); q++)
+    for (size_t q = 0; q < n_fast_segs; q++)
         s += "XT_GEN_FN void fast_seg_" + std::to_string(q) + "(xt::FState &p) {\n    (void)p;\n" +
              cs.fast_segs[q] + "}\n\n";
     // a segment's records that address the program (relative literal code
@@ -951,6 +994,7 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
          "    const int32_t *__restrict__ rec;\n"
          "    const int64_t *__restrict__ entry;\n"
          "    const double *__restrict__ prog;\n";
+    s += "    static constexpr bool kSegments = true;\n";
     if (cs.keyed_pc)
         s += "    struct Key { int32_t r; int64_t pc; };\n"
              "    XT_HD Key key(int64_t e) const { return Key{xt::cptr(rec)[e], xt::cptr(entry)[e]}; }\n";
@@ -981,31 +1025,48 @@ std::string emit_code_set(const CodeSet &cs, uint32_t options, const char *what)
              "(p, m, prog, rp, c); break;\n";
     s += "        default: p.state = -999; break;\n"
          "        }\n"
-         "    }\n"
-         "    /* the units of xt_fast.h */\n"
-         "    XT_HD void fast_segment(xt::FState &p, Key k) const {\n"
-         "        switch (" + kr + " >> " + std::to_string(XT_KEY_SEG_SHIFT) + ") {\n";
-    for (size_t q = 0; q < cs.segs.size(); q++)
-        s += "        case " + std::to_string(q + 1) + ": fast_seg_" + std::to_string(q) +
-             "(p); break;\n";
-    s += "        default: p.bad = true; break;\n"
-         "        }\n"
-         "    }\n"
-         "    XT_HD void fast(xt::FState &p, Key k) const {\n" + rp +
-         "        switch (" + kr + " & " + std::to_string(XT_KEY_REC_MASK) + ") {\n";
-    for (size_t r = 0; r < cs.body.size(); r++)
-        s += "        case " + std::to_string(r) + ": fast_" + std::to_string(r) +
-             "(p, rp); break;\n";
-    s += "        default: p.bad = true; break;\n"
-         "        }\n"
-         "    }\n"
-         "};\n";
+         "    }\n";
+    if (cs.units) {
+        s += "    /* the units of xt_fast.h */\n"
+             "    XT_HD void fast_segment(xt::FState &p, Key k) const {\n"
+             "        switch (" + kr + " >> " + std::to_string(XT_KEY_SEG_SHIFT) + ") {\n";
+        for (size_t q = 0; q < n_fast_segs; q++)
+            s += "        case " + std::to_string(q + 1) + ": fast_seg_" + std::to_string(q) +
+                 "(p); break;\n";
+        s += "        default: p.bad = true; break;\n"
+             "        }\n"
+             "    }\n"
+             "    XT_HD void fast(xt::FState &p, Key k) const {\n" + rp +
+             "        switch (" + kr + " & " + std::to_string(XT_KEY_REC_MASK) + ") {\n";
+        for (size_t r = 0; r < n_fast; r++)
+            s += "        case " + std::to_string(r) + ": fast_" + std::to_string(r) +
+                 "(p, rp); break;\n";
+        s += "        default: p.bad = true; break;\n"
+             "        }\n"
+             "    }\n";
+    }
+    s += "};\n";
     return s;
 }
 
 }  // namespace
 
 namespace {
+
+/* The call that tracks the chi == 1 particle i of a kernel (device) or of the
+   host build: with the loop over units every lane of a wave takes part. */
+std::string track_call(bool units, bool backtrack, bool device, const std::string &pad,
+                       const std::string &runner, const std::string &args) {
+    const std::string in = "\n" + pad + "    ";
+    if (units)
+        return pad + "xt::track_particle_units<" + (backtrack ? "true" : "false") + ">(" +
+               (device ? "P" : "*P") + ", i, " + (device ? "alive" : "true") + "," + in + runner +
+               ", c," + in + args + ", " + (device ? "xt::kernarg()" : "mon") + ");\n";
+    return (device ? pad + "const xt::MonRef mon = xt::kernarg();\n" + pad + "if (alive)\n    "
+                   : std::string()) +
+           pad + "xt::track_particle_loop<true, false>(" + (device ? "*mon.P" : "*P") + ", i," +
+           in + runner + ", c," + in + args + ", mon);\n";
+}
 
 int line_source(const std::vector<int64_t> &entry, const std::vector<double> &prog,
                 int32_t waves_per_eu, uint32_t options, std::string &src,
@@ -1015,8 +1076,12 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
     const int st = build_code_set({&entry}, {&prog}, false, cs, recs, err);
     if (st != XTM_OK) return st;
     rec_of_elem = std::move(recs[0]);
+    // backwards there is no loop over compiled general code
+    if (backtrack) cs.units = true;
     std::string s = emit_code_set(cs, options, "line code");
-    const std::string bt = backtrack ? "<true>" : "<false>";
+    const std::string run = "xt_gen::Runner{rec, entry, prog}";
+    const std::string args = "num_turns, ele_start, num_ele_track, flag_end_turn_actions, "
+                             "flag_reset_s, flag_monitor";
     s += "}  // namespace xt_gen\n\n";
     s += "#if defined(__HIPCC__)\n";
     char occ[128];
@@ -1032,11 +1097,8 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
          "    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;\n"
          "    const xt::TrackCtx c{flags, line_length, P.q0, P.t_sim, num_ele_line};\n"
          "    // chi == 1 particles; the interpreter kernel tracks the others\n"
-         "    const bool alive = i < P.capacity && P.state[i] > 0 && P.chi[i] == 1.0;\n"
-         "    xt::track_particle_units" + bt + "(P, i, alive, xt_gen::Runner{rec, entry, prog}, c,\n"
-         "                             num_turns, ele_start, num_ele_track,\n"
-         "                             flag_end_turn_actions, flag_reset_s, flag_monitor,\n"
-         "                             xt::kernarg());\n"
+         "    const bool alive = i < P.capacity && P.state[i] > 0 && P.chi[i] == 1.0;\n" +
+         track_call(cs.units, backtrack, true, "    ", run, args) +
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over all particles\n"
@@ -1052,16 +1114,11 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
          "    const xt::MonRef mon{M ? M : &m0, P};\n"
          "    for (int64_t i = 0; i < P->capacity; i++) {\n"
          "        if (!(P->state[i] > 0)) continue;\n"
-         "        if (P->chi[i] == 1.0)\n"
-         "            xt::track_particle_units" + bt + "(*P, i, true, xt_gen::Runner{rec, entry, prog}, c,\n"
-         "                                     num_turns, ele_start, num_ele_track,\n"
-         "                                     flag_end_turn_actions, flag_reset_s,\n"
-         "                                     flag_monitor, mon);\n"
+         "        if (P->chi[i] == 1.0)\n" +
+         track_call(cs.units, backtrack, false, "            ", run, args) +
          "        else\n"
          "            xt::track_particle_loop_cold<false>(*P, i, xt::ProgramRunner{entry, prog},\n"
-         "                                     c, num_turns, ele_start, num_ele_track,\n"
-         "                                     flag_end_turn_actions, flag_reset_s,\n"
-         "                                     flag_monitor, mon);\n"
+         "                c, " + args + ", mon);\n"
          "    }\n"
          "}\n"
          "#endif\n";
@@ -1114,11 +1171,11 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "    const xt::TrackCtx c{flags, xt::cptr(lengths)[b.line], P.q0, P.t_sim, ne};\n"
          "    // chi == 1 particles; the interpreter batch kernel tracks the others\n"
          "    const bool alive = (int32_t)threadIdx.x < b.count && P.state[i] > 0 &&\n"
-         "                       P.chi[i] == 1.0;\n"
-         "    xt::track_particle_units<false>(P, i, alive, xt_gen::Runner{xt::cptr(recs)[b.line],\n"
-         "                             xt::cptr(entries)[b.line], xt::cptr(progs)[b.line]}, c,\n"
-         "                             num_turns, 0, (int32_t)ne, 1, 1, flag_monitor,\n"
-         "                             xt::kernarg());\n"
+         "                       P.chi[i] == 1.0;\n" +
+         track_call(cs.units, false, true, "    ",
+                    "xt_gen::Runner{xt::cptr(recs)[b.line], xt::cptr(entries)[b.line], "
+                    "xt::cptr(progs)[b.line]}",
+                    "num_turns, 0, (int32_t)ne, 1, 1, flag_monitor") +
          "}\n"
          "#else\n"
          "// host build (tests): the same per-particle body over the blocks\n"
@@ -1133,10 +1190,10 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
          "        const xt::MonRef mon{nullptr, P};\n"
          "        for (int64_t i = b.first; i < b.first + b.count; i++) {\n"
          "            if (!(P->state[i] > 0)) continue;\n"
-         "            if (P->chi[i] == 1.0)\n"
-         "                xt::track_particle_units<false>(*P, i, true,\n"
-         "                    xt_gen::Runner{recs[b.line], entries[b.line], progs[b.line]}, c,\n"
-         "                    num_turns, 0, (int32_t)ne, 1, 1, 0, mon);\n"
+         "            if (P->chi[i] == 1.0)\n" +
+         track_call(cs.units, false, false, "                ",
+                    "xt_gen::Runner{recs[b.line], entries[b.line], progs[b.line]}",
+                    "num_turns, 0, (int32_t)ne, 1, 1, 0") +
          "            else\n"
          "                xt::track_particle_loop_cold<false>(*P, i,\n"
          "                    xt::ProgramRunner{entries[b.line], progs[b.line]}, c, num_turns, 0,\n"

@@ -353,6 +353,13 @@ XT_HD void f_xy_shift(FState &p, const double ax, const double ay) {
     p.y = p.y + ay;
 }
 
+/* op_s_shift of xt_ops.h */
+XT_HD void f_s_shift(FState &p, const double ds) {
+    f_drift_exact(p, ds);
+    p.zeta = p.zeta + (-ds);
+    p.s = p.s + (-ds);
+}
+
 XT_HD void f_s_rot(FState &p, const double sin_z, const double cos_z) {
     const double x = p.x, y = p.y, px = p.px, py = p.py;
     p.x = cos_z * x + sin_z * y;

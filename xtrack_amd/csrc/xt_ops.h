@@ -1398,8 +1398,9 @@ XT_HD_COLD void feature_hook(const xtm_features *F, const int64_t i, const doubl
    at_element: the reference adds 1 after every element the particle
    survives and sets 0 at the end of a turn; here at_element = base + e at
    element e, with base updated at the end of each turn.
-   run(p, m, run.key(e), c) tracks element e: the program interpreter (the
-   compiled code's loop is track_particle_units in xt_fast.h).
+   run(p, m, run.key(e), c) tracks element e: the program interpreter, or
+   compiled code of lines whose elements mostly have no unit code (the loop of
+   the others is track_particle_units in xt_fast.h).
    CHI1: the particle's chi is exactly 1.0 and the element code sees the
    constant, so products with chi fold away (chi * k == k exactly) instead
    of being evaluated, or hoisted out of the loops as per-particle values
@@ -1451,12 +1452,27 @@ XT_HD void track_particle_loop(const xtm_particles &P, int64_t i, const Runner &
                current element's arithmetic */
             typename Runner::Key key{};
             if (ele_start < ele_stop) key = run.key(ele_start);
-            for (int64_t e = ele_start; e < ele_stop; e++) {
-                const typename Runner::Key next = run.key(e + 1 < ele_stop ? e + 1 : e);
+            for (int64_t e = ele_start; e < ele_stop;) {
+                /* a runner with segments tracks a run of n consecutive
+                   elements in one call (not with element-by-element
+                   records) and returns the position j in the run of the
+                   element where the particle was lost */
+                int64_t n = 1, j = 0;
+                if constexpr (Runner::kSegments) {
+                    const int32_t span = Runner::span(key);
+                    if (span > 1 && flag_monitor != 2 && e + span <= ele_stop) n = span;
+                }
+                const typename Runner::Key next = run.key(e + n < ele_stop ? e + n : e);
                 if (flag_monitor == 2) XT_MONITOR_RECORD(base + e);
-                run(p, m, key, c);
+                if constexpr (Runner::kSegments) {
+                    if (n > 1) j = run.segment(p, m, key, c, e);
+                    else run(p, m, key, c);
+                } else {
+                    run(p, m, key, c);
+                }
                 if (c.freeze_long()) p.zeta = p.get(XS_ZETA0);
-                if (p.state <= 0) { e_lost = e; break; }
+                if (p.state <= 0) { e_lost = e + j; break; }
+                e += n;
                 key = next;
             }
             if (e_lost >= 0) break;
@@ -1509,6 +1525,7 @@ struct ProgramRunner {
     const int64_t *__restrict__ entry;
     const double *__restrict__ prog;
     using Key = int64_t;
+    static constexpr bool kSegments = false;
     XT_HD Key key(int64_t e) const { return cptr(entry)[e]; }
     XT_HD void operator()(PState<double> &p, const PRef &m, Key pc, const TrackCtx &c) const {
         run_element(p, m, cptr(prog), uniform(pc), c);
