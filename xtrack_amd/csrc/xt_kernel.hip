@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <string>
@@ -445,14 +446,21 @@ static const LineCode *backtrack_code(xtm_line *L, hipStream_t stream) {
     if (L->bt.kernel) return &L->bt;
     if (L->bt_waves == 0) return nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-        return nullptr;
-    const std::vector<int64_t> rev(L->entry_bt.rbegin(), L->entry_bt.rend());
-    if (load_line_code(L, rev, L->bt_waves, 0, true, L->bt) != XTM_OK) {
-        L->bt_waves = 0;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
         return nullptr;
     }
-    return &L->bt;
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    try {
+        const std::vector<int64_t> rev(L->entry_bt.rbegin(), L->entry_bt.rend());
+        if (load_line_code(L, rev, L->bt_waves, 0, true, L->bt) == XTM_OK) return &L->bt;
+    } catch (const std::exception &) {
+        // out of memory: as code that does not load
+    }
+    // the error that the failed call left is not the interpreter launch's
+    (void)hipGetLastError();
+    L->bt_waves = 0;
+    return nullptr;
 }
 
 int32_t xtm_line_is_specialized(const xtm_line *L) { return (L && L->code.kernel) ? 1 : 0; }
