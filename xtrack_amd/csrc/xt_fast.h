@@ -569,10 +569,11 @@ XT_HD void track_particle_units(const xtm_particles &P, const int64_t i, bool al
             e += n;
             key = next;
         }
-        if (flag_monitor == 2) {
+        /* backwards also a record of flag_monitor 1, as in track_particle_loop */
+        if (flag_monitor == 2 || (BT && flag_monitor == 1)) {
             store_axay();
             FState q = p;
-            if (alive) general(q, key, ele_stop, 0, 2);
+            if (alive) general(q, key, ele_stop, 0, BT ? flag_monitor : 2);
         }
         if (!BT && flag_end_turn_actions > 0) {
             at_turn += 1;
