@@ -1,0 +1,44 @@
+"""Which library calls the network's methods make: the library's entry points
+are recorded and CPU tensors stand for device tensors, so that the choice
+between the library's steps and the layered pass is seen without a GPU."""
+import pytest
+import torch
+
+from xtrack_amd import surrogate
+
+
+class _Recorder:
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append((name, args))
+            return 4096 if name == 'xtm_mlp_workspace_bytes' else 0
+        return call
+
+    def names(self):
+        out = [n for n, _ in self.calls if n != 'xtm_mlp_workspace_bytes']
+        self.calls.clear()
+        return out
+
+
+@pytest.fixture
+def lib(monkeypatch):
+    rec = _Recorder()
+    monkeypatch.setattr(surrogate._native, 'load', lambda: rec)
+    monkeypatch.setattr(surrogate, '_stream', lambda dev: None)
+    monkeypatch.setattr(torch.Tensor, 'is_cuda', property(lambda t: True))
+    return rec
+
+
+def _net(sizes=surrogate.SIZES):
+    return surrogate.MLP(device='cpu', sizes=sizes)
+
+
+def test_layers_beyond_the_limits_of_the_step(lib):
+    net = _net((4, 2 ** 20 + 1, 1))
+    net.forward(torch.zeros(1, 4), keep=True)
+    assert lib.names() == ['xtm_gemm_bf16'] * 2
+    _net((4, 32, 1)).forward(torch.zeros(1, 4), keep=True)
+    assert lib.names() == ['xtm_mlp_train_forward']

@@ -169,11 +169,13 @@ class MLP:
 
     def _native_step(self, x):
         """Whether the library's training step takes this network (at most 8
-        layers, one output, contiguous FP32 parameters) and the rows of x."""
+        layers of at most 2^20 values, one output, contiguous FP32 parameters)
+        and the rows of x."""
         torch = _t()
         ps = self.W + self.b
         shapes = list(zip(self.sizes[:-1], self.sizes[1:])) + [(n,) for n in self.sizes[1:]]
-        return (len(self.W) <= 8 and self.sizes[-1] == 1 and len(x) > 0 and x.is_cuda
+        return (len(self.W) <= 8 and self.sizes[-1] == 1 and 0 < len(x) < 2 ** 31 and x.is_cuda
+                and all(1 <= n <= 2 ** 20 for n in self.sizes)
                 and all(p.dtype == torch.float32 and p.device == x.device and p.is_contiguous()
                         for p in ps) and [tuple(p.shape) for p in ps] == shapes)
 
