@@ -42,3 +42,12 @@ def test_layers_beyond_the_limits_of_the_step(lib):
     assert lib.names() == ['xtm_gemm_bf16'] * 2
     _net((4, 32, 1)).forward(torch.zeros(1, 4), keep=True)
     assert lib.names() == ['xtm_mlp_train_forward']
+
+
+@pytest.mark.parametrize('shape', [(2, 16, 3), (16,), (3, 16, 16)], ids=str)
+@pytest.mark.parametrize('keep', [False, True])
+def test_inputs_that_are_not_rows_are_refused(lib, shape, keep):
+    for sizes in (surrogate.SIZES, (16, 32, 1)):
+        with pytest.raises(ValueError, match='2-D'):
+            _net(sizes).forward(torch.zeros(shape), keep=keep)
+    assert not lib.names()

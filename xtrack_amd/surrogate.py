@@ -150,7 +150,7 @@ class MLP:
         torch = _t()
         if not keep and self._one_kernel(x):
             return self._run_one_kernel(x)
-        if not self._native_step(x) or x.shape[1] != self.sizes[0]:
+        if x.dim() != 2 or x.shape[1] != self.sizes[0] or not self._native_step(x):
             return self._forward_layers(x, keep)
         lib = _native.load()
         B = len(x)
