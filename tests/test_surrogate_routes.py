@@ -51,3 +51,24 @@ def test_inputs_that_are_not_rows_are_refused(lib, shape, keep):
         with pytest.raises(ValueError, match='2-D'):
             _net(sizes).forward(torch.zeros(shape), keep=keep)
     assert not lib.names()
+
+
+def test_prediction_with_scalar_and_tensor_normalisation(lib):
+    """Means and deviations that broadcast as tensor operations do, numbers
+    and device scalars among them."""
+    x = torch.zeros(5, 16)
+    net = _net()
+    net.x_mean, net.x_std = torch.zeros(16), torch.ones(16)
+    net.predict(x)
+    assert lib.names() == ['xtm_mlp_forward']
+    for mean, std in ((0.0, 1.0), (torch.zeros(()), torch.ones(())), (torch.zeros(16), 2.0)):
+        net.x_mean, net.x_std = mean, std
+        assert net.predict(x).shape == (5,)
+        (name, args), = [c for c in lib.calls if c[0] == 'xtm_mlp_forward']
+        assert args[1] is None and args[8] == 0      # normalised before and after
+        lib.names()
+    net.x_mean, net.x_std = torch.zeros(16), torch.ones(16)
+    net.y_mean, net.y_std = torch.zeros(()), torch.ones(())
+    assert net.predict(x).shape == (5,)
+    (name, args), = [c for c in lib.calls if c[0] == 'xtm_mlp_forward']
+    assert args[8] == 0

@@ -21,6 +21,7 @@ error is measured against.
 """
 import ctypes
 import math
+import numbers
 import time
 
 import numpy as np
@@ -41,6 +42,11 @@ def _ptr(t):
 
 def _pointers(tensors):
     return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _numbers(*values):
+    """Whether all of them are numbers of the host."""
+    return all(isinstance(v, numbers.Real) for v in values)
 
 
 def _stream(dev):
@@ -122,7 +128,8 @@ class MLP:
         throughout, on one device; everything else goes layer by layer."""
         torch = _t()
         ts = [x, *vectors, *self.W, *self.b]
-        return (self.sizes == SIZES and x.dim() == 2 and x.shape[1] == SIZES[0] and len(x) > 0
+        return (self.sizes == SIZES and all(isinstance(t, torch.Tensor) for t in ts)
+                and x.dim() == 2 and x.shape[1] == SIZES[0] and len(x) > 0
                 and all(t.dtype == torch.float32 and t.device == x.device for t in ts)
                 and x.is_cuda and all(t.is_contiguous() for t in self.W + self.b)
                 and all(tuple(t.shape) == (SIZES[0],) for t in vectors)
@@ -341,7 +348,8 @@ class MLP:
 
     def predict(self, x, batch=65536):
         torch = _t()
-        if self._one_kernel(x, self.x_mean, self.x_std):
+        if (_numbers(self.y_mean, self.y_std)
+                and self._one_kernel(x, self.x_mean, self.x_std)):
             return self._run_one_kernel(x, self.x_mean, self.x_std, self.y_std, self.y_mean)
         xn = (x - self.x_mean) / self.x_std
         out = [self.forward(xn[s:s + batch]) for s in range(0, len(xn), batch)]
