@@ -72,3 +72,26 @@ def test_prediction_with_scalar_and_tensor_normalisation(lib):
     assert net.predict(x).shape == (5,)
     (name, args), = [c for c in lib.calls if c[0] == 'xtm_mlp_forward']
     assert args[8] == 0
+
+
+@pytest.mark.parametrize('change', ['strides', 'dtype', 'shape'])
+def test_weights_changed_between_the_passes(lib, change):
+    """The backward pass looks at the weights that it is given."""
+    net = _net((16, 32, 32, 1))
+    x, dout = torch.zeros(7, 16), torch.ones(7)
+    net.forward(x, keep=True)
+    net.backward(dout)
+    assert lib.names() == ['xtm_mlp_train_forward', 'xtm_mlp_train_backward']
+    net.forward(x, keep=True)
+    lib.names()
+    w = net.W[1]
+    net.W[1] = {'strides': lambda: w.t().contiguous().t(), 'dtype': lambda: w.double(),
+                'shape': lambda: w[:, :8].contiguous()}[change]()
+    if change == 'shape':
+        with pytest.raises(ValueError, match='inner dimensions'):
+            net.backward(dout)
+        return
+    gw, gb = net.backward(dout)
+    assert lib.names() == ['xtm_gemm_bf16'] * 5
+    assert [tuple(g.shape) for g in gw] == [(16, 32), (32, 32), (32, 1)]
+    assert [tuple(g.shape) for g in gb] == [(32,), (32,), (1,)]

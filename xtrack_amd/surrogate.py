@@ -204,9 +204,19 @@ class MLP:
             self._cache = (acts, zs)
         return zs[-1][:, 0]
 
+    def _layer_cache(self):
+        """The forward pass's activations and products by layer."""
+        if len(self._cache) == 2:
+            return self._cache
+        xb, z, h = self._cache
+        widths = self.sizes[1:-1]
+        cut = [len(xb) * n for n in widths]
+        return ([xb] + [v.view(-1, n) for v, n in zip(h.split(cut), widths)],
+                [v.view(-1, n) for v, n in zip(z.split(cut), widths)])
+
     def _backward_layers(self, dout):
-        """The backward pass after _forward_layers."""
-        acts, zs = self._cache
+        """The backward pass product by product."""
+        acts, zs = self._layer_cache()
         n = len(self.W)
         dz = dout.reshape(-1, 1).to(_t().float32)
         gW, gb = [None] * n, [None] * n
@@ -235,6 +245,8 @@ class MLP:
             return self._backward_layers(dout)
         lib = _native.load()
         xb, z, h = self._cache
+        if not self._native_step(xb):      # the weights are others than in the forward pass
+            return self._backward_layers(dout)
         B, n = len(xb), len(self.W)
         dout = dout.reshape(-1).to(torch.float32).contiguous()
         if len(dout) != B:
