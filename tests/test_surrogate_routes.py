@@ -95,3 +95,19 @@ def test_weights_changed_between_the_passes(lib, change):
     assert lib.names() == ['xtm_gemm_bf16'] * 5
     assert [tuple(g.shape) for g in gw] == [(16, 32), (32, 32), (32, 1)]
     assert [tuple(g.shape) for g in gb] == [(32,), (32,), (1,)]
+
+
+def test_adam_with_a_tensor_learning_rate(lib):
+    """A learning rate on the device (changed between graph replays) is not
+    read by the host."""
+    net = _net((4, 8, 1))
+    g = [torch.ones_like(w) for w in net.W], [torch.ones_like(b) for b in net.b]
+    net.adam_step(*g, lr=1e-3)
+    assert lib.names() == ['xtm_adam_step']
+    before = [p.clone() for p in net.W + net.b]
+    net.adam_step(*g, lr=torch.tensor(0.25))
+    assert not lib.names()
+    # the first recorded step changed no moment: m = 0.1, v = 0.001, t = 2
+    step = 0.25 * (0.1 / (1 - 0.9 ** 2)) / ((0.001 / (1 - 0.999 ** 2)) ** 0.5 + 1e-8)
+    for p, q in zip(net.W + net.b, before):
+        assert torch.allclose(q - p, torch.full_like(p, step), rtol=1e-4, atol=1e-6)

@@ -264,8 +264,9 @@ class MLP:
 
     def adam_step(self, gW, gb, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
         """One Adam update of the weights and biases in place (FP32 arrays on
-        the device: in one kernel).  The step count lives on the device, so that the update can be captured
-        in a HIP graph and replayed."""
+        the device and rates that are numbers: in one kernel).  The step count
+        lives on the device, so that the update can be captured in a HIP graph
+        and replayed."""
         torch = _t()
         params, grads = self.W + self.b, list(gW) + list(gb)
         if self._adam is None:
@@ -274,7 +275,8 @@ class MLP:
                           'v': [torch.zeros_like(p) for p in params]}
         st = self._adam
         st['t'].add_(1.0)
-        if (len(params) <= 16 and len(grads) == len(params) and st['t'].is_cuda
+        if (_numbers(lr, beta1, beta2, eps) and len(params) <= 16
+                and len(grads) == len(params) and st['t'].is_cuda
                 and all(t.dtype == torch.float32 and t.device == st['t'].device
                         and t.is_contiguous() and t.shape == p.shape
                         for p, *ts in zip(params, grads, st['m'], st['v']) for t in (p, *ts))):
