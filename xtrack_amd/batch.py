@@ -119,6 +119,8 @@ class BatchTracker:
         big.start_tracking_at_element = -1
         if self._on_device(particles_list):
             import torch
+            # the sets may have been written on any stream
+            torch.cuda.synchronize(self.device)
             big._arrays = {}
             for nn in ref._arrays:
                 parts = [pp._arrays[nn] for pp in particles_list]
@@ -144,9 +146,11 @@ class BatchTracker:
         """Each set gets its part of the tracked set (on the device: its range
         of the joined arrays)."""
         if self._on_device(particles_list):
+            import torch
             for nn, vv in big._arrays.items():
                 for k, pp in enumerate(particles_list):
                     pp._arrays[nn] = vv[starts[k]:starts[k + 1]]
+            torch.cuda.synchronize(self.device)      # and may be read on any
             return
         host = big.to_numpy()
         for k, pp in enumerate(particles_list):
