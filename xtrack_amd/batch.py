@@ -47,6 +47,12 @@ CANDIDATES = tuple((bs, w) for bs in BLOCK_SIZES for w in (3, 4, 5))
 COMPILED_CANDIDATES = tuple((bs, 5) for bs in BLOCK_SIZES)
 
 
+def _rows(names, dtype, buf):
+    """The rows of a buffer as the named fields."""
+    rows = buf.unbind()
+    return zip(names, rows if buf.dtype == dtype else [r.view(dtype) for r in rows])
+
+
 class BatchTracker:
     def __init__(self, lines, device='cuda:0', compile='auto', waves_per_eu=0):
         import torch
@@ -121,14 +127,19 @@ class BatchTracker:
             import torch
             # the sets may have been written on any stream
             torch.cuda.synchronize(self.device)
-            big._arrays = {}
-            for nn in ref._arrays:
-                parts = [pp._arrays[nn] for pp in particles_list]
-                if parts[0].dtype == torch.uint32:     # no unsigned concatenation
-                    big._arrays[nn] = torch.cat([v.view(torch.int32) for v in parts]).view(
-                        torch.uint32)
-                else:
-                    big._arrays[nn] = torch.cat(parts)
+            # the fields of one type are the rows of one buffer
+            big._joined = []
+            for dtype in dict.fromkeys(vv.dtype for vv in ref._arrays.values()):
+                names = [nn for nn, vv in ref._arrays.items() if vv.dtype == dtype]
+                # no unsigned concatenation
+                held = torch.int32 if dtype == torch.uint32 else dtype
+                buf = torch.empty((len(names), big._capacity), dtype=held, device=self.device)
+                for nn, row in zip(names, buf.unbind()):
+                    parts = [pp._arrays[nn] for pp in particles_list]
+                    torch.cat(parts if held == dtype else [v.view(held) for v in parts], out=row)
+                big._joined.append((names, dtype, buf))
+            rows = {nn: row for joined in big._joined for nn, row in _rows(*joined)}
+            big._arrays = {nn: rows[nn] for nn in ref._arrays}
             big._device = self.device
             return big, starts
         hosts = [pp.to_numpy() for pp in particles_list]
@@ -143,13 +154,16 @@ class BatchTracker:
         return all(pp.device == self.device for pp in particles_list)
 
     def _split(self, big, starts, particles_list):
-        """Each set gets its part of the tracked set (on the device: its range
-        of the joined arrays)."""
+        """Each set gets its part of the tracked set: on the device, copies of
+        its columns of the joined buffers, which the set alone holds."""
         if self._on_device(particles_list):
             import torch
-            for nn, vv in big._arrays.items():
-                for k, pp in enumerate(particles_list):
-                    pp._arrays[nn] = vv[starts[k]:starts[k + 1]]
+            for k, pp in enumerate(particles_list):
+                part = dict.fromkeys(big._arrays)
+                for names, dtype, buf in big._joined:
+                    part.update(_rows(names, dtype, buf[:, starts[k]:starts[k + 1]].clone(
+                        memory_format=torch.contiguous_format)))
+                pp._arrays = part
             torch.cuda.synchronize(self.device)      # and may be read on any
             return
         host = big.to_numpy()
