@@ -19,6 +19,8 @@ def _zero_particles(n_records, device=None):
         out._device = _device_of(device)
         buf = torch.zeros(n * sum(np.dtype(tt).itemsize for tt, _ in per_particle_vars),
                           dtype=torch.uint8, device=out._device)
+        # the records may be written on another stream than the fill's
+        torch.cuda.current_stream(out._device).synchronize()
         out._arrays, at = {}, 0
         # the 8-byte fields come first, so every field is aligned
         for tt, nn in per_particle_vars:
