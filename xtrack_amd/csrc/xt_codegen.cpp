@@ -665,10 +665,22 @@ std::string both(const std::string &general, const std::string &unit) {
     return general + '\n' + unit;
 }
 
+/* with_units: general and unit code of every function; else general code
+   alone, for the element loop. */
 int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                    const std::vector<const std::vector<double> *> &progs, bool keyed_pc,
-                   CodeSet &cs, std::vector<std::vector<int32_t>> &recs, std::string &err) {
+                   bool with_units, CodeSet &cs, std::vector<std::vector<int32_t>> &recs,
+                   std::string &err) {
     const size_t nl = entries.size();
+    cs = CodeSet();
+    // a program that the unit generator does not read has no unit code
+    auto unit = [&](FastGen &f, int64_t pc) {
+        if (with_units && !f.record(pc)) {
+            f.direct = true;
+            f.gain = -200;
+        }
+        return with_units ? f.body() : std::string();
+    };
     // distinct records of each line and their element counts
     std::vector<std::map<int64_t, int64_t>> uses(nl);
     int64_t n_distinct = 0;
@@ -699,22 +711,21 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
             Gen g(*progs[l], pu.first, false, !all_literal);
             Gen gs(*progs[l], pu.first, true);
             FastGen f(*progs[l], false), fs(*progs[l], true);
-            if (!g.record(pu.first) || !gs.record(pu.first) || !f.record(pu.first) ||
-                !fs.record(pu.first)) {
+            if (!g.record(pu.first) || !gs.record(pu.first)) {
                 err = "cannot generate code for line " + std::to_string(l) +
                       " at program offset " + std::to_string(pu.first);
                 return XTM_ERR_ARG;
             }
-            const std::string unit = f.body();
-            auto ins = lits.emplace(both(g.out, unit), Literal());
+            const std::string fast = unit(f, pu.first), fast_struct = unit(fs, pu.first);
+            auto ins = lits.emplace(both(g.out, fast), Literal());
             Literal &v = ins.first->second;
             if (ins.second) {
                 v.general = g.out;
-                v.unit = unit;
+                v.unit = fast;
                 // a structure is its general and its unit code: records of
                 // one op sequence differ in the latter where a form depends
                 // on the ranges of their constants
-                v.structure = both(gs.out, fs.body());
+                v.structure = both(gs.out, fast_struct);
                 v.small = !g.heavy && g.cost <= kSmallCost;
                 v.weight = f.weight(v.small);
                 lits_of_struct[v.structure]++;
@@ -731,7 +742,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     // 100 RF multipoles 1016 / 3702 against 1165 / 5059; 60 quadrupoles that
     // are off among 60 that are on 278 / 895 against 215 / 710, 108 thin kicks
     // with 12 rotated ones 61 / 194 against 47 / 151.
-    cs.units = gain >= 0;
+    cs.units = with_units && gain >= 0;
     // A structure that the set holds with many different constants (the
     // bends of ring variants with different cell counts) gets one structure
     // function rather than a literal copy per constant set.
@@ -765,12 +776,12 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
             }
             Gen g(*progs[l], pu.first, true);
             FastGen f(*progs[l], true);
-            if (!g.record(pu.first) || !f.record(pu.first)) {
+            if (!g.record(pu.first)) {
                 err = "cannot generate code for line " + std::to_string(l) +
                       " at program offset " + std::to_string(pu.first);
                 return XTM_ERR_ARG;
             }
-            const std::string fast = f.body();
+            const std::string fast = unit(f, pu.first);
             auto ins = fn_of_struct.emplace(both(g.out, fast), (int32_t)cs.body.size());
             if (ins.second) {
                 cs.body.push_back(g.out);
@@ -808,11 +819,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                 shared[k] = shared[k] && wbits((*progs[rc.first])[rc.second + k]) ==
                                              wbits((*progs[l0])[pc0 + k]);
         FastGen f(*progs[l0], true, &shared);
-        if (!f.record(pc0)) {
-            err = "cannot generate unit code at program offset " + std::to_string(pc0);
-            return XTM_ERR_ARG;
-        }
-        cs.fast[kv.first] = f.body();
+        cs.fast[kv.first] = unit(f, pc0);
     }
 
     // Segments: runs of consecutive cheap literal records (drifts,
@@ -922,12 +929,8 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         cs.segs.push_back(r.second);
         const Chunk &ch = where[r.second];
         FastGen f(*progs[std::get<0>(ch)], false);
-        for (size_t j = 0; j < std::get<2>(ch); j++)
-            if (!f.record((*entries[std::get<0>(ch)])[std::get<1>(ch) + j])) {
-                err = "cannot generate code for a segment of line " +
-                      std::to_string(std::get<0>(ch));
-                return XTM_ERR_ARG;
-            }
+        for (size_t j = 0; with_units && j < std::get<2>(ch); j++)
+            f.direct |= !f.record((*entries[std::get<0>(ch)])[std::get<1>(ch) + j]);
         cs.fast_segs.push_back(f.body());
     }
     for (auto &ch : chunks) {
@@ -937,6 +940,19 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
                                                   ((int32_t)std::get<2>(ch) << XT_KEY_SPAN_SHIFT);
     }
     return XTM_OK;
+}
+
+/* The code set for tracking: with units where it compiles with them and gains
+   by them.  Functions are shared by records whose general and unit code
+   agree, so a set near XT_CODEGEN_MAX_RECORDS functions may fit without units
+   only. */
+int choose_code_set(const std::vector<const std::vector<int64_t> *> &entries,
+                    const std::vector<const std::vector<double> *> &progs, bool keyed_pc,
+                    CodeSet &cs, std::vector<std::vector<int32_t>> &recs, std::string &err) {
+    const int st = build_code_set(entries, progs, keyed_pc, true, cs, recs, err);
+    if (st == XTM_OK && cs.units) return st;
+    if (st != XTM_OK && st != XTM_ERR_UNSUPPORTED) return st;
+    return build_code_set(entries, progs, keyed_pc, false, cs, recs, err);
 }
 
 /* The functions, segments and element runner of a code set, in namespace
@@ -1073,11 +1089,13 @@ int line_source(const std::vector<int64_t> &entry, const std::vector<double> &pr
                 std::vector<int32_t> &rec_of_elem, std::string &err, bool backtrack) {
     CodeSet cs;
     std::vector<std::vector<int32_t>> recs;
-    const int st = build_code_set({&entry}, {&prog}, false, cs, recs, err);
-    if (st != XTM_OK) return st;
-    rec_of_elem = std::move(recs[0]);
     // backwards there is no loop over compiled general code
+    const int st = backtrack
+                       ? build_code_set({&entry}, {&prog}, false, true, cs, recs, err)
+                       : choose_code_set({&entry}, {&prog}, false, cs, recs, err);
+    if (st != XTM_OK) return st;
     if (backtrack) cs.units = true;
+    rec_of_elem = std::move(recs[0]);
     std::string s = emit_code_set(cs, options, "line code");
     const std::string run = "xt_gen::Runner{rec, entry, prog}";
     const std::string args = "num_turns, ele_start, num_ele_track, flag_end_turn_actions, "
@@ -1148,7 +1166,7 @@ int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &en
                              std::vector<std::vector<int32_t>> &recs, std::string &err) {
     CodeSet cs;
     // the batch kernel's runner reads each element's program offset
-    const int st = build_code_set(entries, progs, true, cs, recs, err);
+    const int st = choose_code_set(entries, progs, true, cs, recs, err);
     if (st != XTM_OK) return st;
     std::string s = emit_code_set(cs, 0, "batch code");
     s += "/* one block of a batch: particles [first, first + count) of line `line` */\n"
