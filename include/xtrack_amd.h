@@ -304,15 +304,15 @@ int64_t xtm_line_num_records(const xtm_line *line);
 /* Compile line code for a created line and use it for every later
  * xtm_track_line call.  Counterpart of the reference's per-line kernel
  * generation and compilation at build_tracker time (xtrack/tracker.py:
- * 544-751, compiled by xobjects): here the generated source has one
- * straight-line function per distinct element record with the record's
- * constants as literals, with the results of the program interpreter's
- * element maps, and is compiled with hiprtc for gfx950.  The code for
- * XTM_FLAG_BACKTRACK is compiled by the first such xtm_track_line call (while
- * the stream is captured that call runs on the interpreter).  waves_per_eu: the
- * kernel's occupancy target (0: the library default).  Returns
- * XTM_ERR_UNSUPPORTED, leaving the interpreter in use, when the line has
- * more distinct records than code is generated for; XTM_ERR_HIP when
+ * 544-751, compiled by xobjects): here the generated source has
+ * straight-line functions of the distinct element records, with the results
+ * of the program interpreter's element maps, and is compiled with hiprtc for
+ * gfx950.  The code for XTM_FLAG_BACKTRACK is compiled by the first such
+ * xtm_track_line call, which then takes seconds (while the stream is captured,
+ * and where that code cannot be loaded, calls run on the interpreter).
+ * waves_per_eu: the kernel's occupancy target (0: the library default).
+ * Returns XTM_ERR_UNSUPPORTED, leaving the interpreter in use, when the line
+ * needs more functions than code is generated for; XTM_ERR_HIP when
  * compilation or loading fails (message in xtm_last_error). */
 int32_t xtm_line_specialize(xtm_line *line, int32_t waves_per_eu);
 
@@ -499,7 +499,8 @@ int32_t xtm_mlp_forward(const float *x, const float *mean, const float *std,
  * w[l] sizes[l] x sizes[l + 1]); wb: scratch for all weights in BF16; z and h:
  * the hidden layers' outputs one after the other, FP32 and BF16; out: B.
  * backward: dout = d loss / d out (B, FP32) to the gradients gw[l], gb[l]; dz
- * and dzb: scratch of the size of z, and of h plus B. */
+ * and dzb: scratch of the size of z, and of h plus B.  Networks of more layers,
+ * or of more than 2^20 values in one, are refused. */
 int32_t xtm_mlp_train_forward(int32_t n, const int64_t *sizes, const uint16_t *xb,
                               const float *const *w, const float *const *b, uint16_t *wb,
                               float *z, uint16_t *h, float *out, int64_t B, void *stream);

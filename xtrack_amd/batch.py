@@ -222,7 +222,7 @@ class BatchTracker:
     def track(self, particles_list, num_turns, turns_per_launch=None, tune=False,
               use_graph=False):
         """Track each particle set through its line for num_turns full turns,
-        in place."""
+        in place; the sets then hold new arrays of their own."""
         import torch
         if num_turns < 0:
             raise ValueError('num_turns must be >= 0')

@@ -4,14 +4,19 @@
 // word and constant of an element from memory and dispatches on the op at
 // run time.  For a line with few distinct element records (a ring is made
 // of a handful of magnet, drift and aperture types repeated thousands of
-// times) this file writes the same op sequence as straight-line calls of
-// the same element functions, with the constants as exact hexadecimal
-// literals, so the device compiler sees constants instead of loads and no
-// per-op dispatch remains; the per-element dispatch becomes one switch on a
-// 32-bit record index.  Folded multipole-kick passes are unrolled with the
-// zero pattern of their coefficients known.  The arithmetic per particle is
-// unchanged: the generated code calls the functions the interpreter calls,
-// with the values the interpreter would load.
+// times) this file writes the same op sequence as straight-line code, with
+// the constants as exact hexadecimal literals, so the device compiler sees
+// constants instead of loads and no per-op dispatch remains; the per-element
+// dispatch becomes one switch on a 32-bit record index.  Folded
+// multipole-kick passes are unrolled with the zero pattern of their
+// coefficients known.
+//
+// There are two codes of a record.  Its general code (Gen) calls the element
+// functions that the interpreter calls, with the values the interpreter would
+// load.  Its unit code (FastGen) runs the maps of xt_fast.h on the state in
+// registers, under guards; a particle that fails one repeats the unit in the
+// general code.  Both give the interpreter's bits.  A line whose elements
+// mostly have no unit code has general code alone.
 #include <cinttypes>
 #include <cmath>
 #include <cstdio>

@@ -18,14 +18,17 @@ constexpr int32_t XT_KEY_SPAN_MASK = 31;
 constexpr int32_t XT_KEY_SEG_SHIFT = 16;
 static_assert(XT_CODEGEN_MAX_RECORDS <= XT_KEY_REC_MASK + 1, "record index must fit its key field");
 
-// Source of a translation unit that tracks the line: one function per
-// distinct element record with the record's constants as literals, an
-// element runner switching on the record index of each element, and (when
-// compiled as HIP) the kernel `xtm_line_kernel`, whose parameters are those
-// of the interpreter kernel with the entry array replaced by `rec`.  The
-// source includes xt_ops.h.  `rec_of_elem[e]` receives the key of element
-// e (its record index and, at the start of a segment of cheap records, the
-// segment fields above).  `waves_per_eu` (> 0) sets the kernel's occupancy target.
+// Source of a translation unit that tracks the line: the functions of the
+// distinct element records (general code and, unless the line tracks faster
+// without, unit code) with the records' constants as literals or read from
+// the program, an element runner switching on the function index of each
+// element, and (when compiled as HIP) the kernel `xtm_line_kernel`: the
+// particle, monitor and feature structs by value, the element keys `rec`,
+// the entry offsets, the program, and the arguments of the call with the
+// number of elements of the line last.  The source includes xt_fast.h.
+// `rec_of_elem[e]` receives the key of element e (its function index and, at
+// the start of a segment of cheap records, the segment fields above).
+// `waves_per_eu` (> 0) sets the kernel's occupancy target.
 // `options`: XTM_SPEC_* bits (XTM_SPEC_FAST_ARITH compiles the element maps
 // with XTM_ARITH_FAST defined).
 // Returns an XTM_* status and sets `err` on failure.
@@ -41,12 +44,13 @@ int xt_generate_backtrack_source(const std::vector<int64_t> &entry,
                                  std::string &err);
 
 // Source of a translation unit that tracks a batch of lines in one launch:
-// one function per distinct element structure (the record code with its
+// literal functions for records that serve several elements, else one
+// function per distinct element structure (the record code with its
 // constants read from the line's program at rp = prog + entry[e], so that
 // the records of all lines that differ only in their constants share one
-// function), an element runner keyed by (structure, program offset), and
+// function), an element runner keyed by (function, program offset), and
 // the kernel `xtm_batch_line_kernel` over a block table (one line per
-// block).  recs[l][e] receives the structure index of element e of line l.
+// block).  recs[l][e] receives the key of element e of line l.
 int xt_generate_batch_source(const std::vector<const std::vector<int64_t> *> &entries,
                              const std::vector<const std::vector<double> *> &progs,
                              int32_t waves_per_eu, std::string &src,

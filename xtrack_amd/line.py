@@ -64,7 +64,8 @@ class Line:
         re-associates the sector-bend polar drift onto reciprocals with a few
         ulp of error per element.  Particles with chi != 1 always run the
         interpreter; backtracking always runs in exact arithmetic, compiled
-        on its first use when the line is compiled."""
+        on its first use when the line is compiled (that call takes seconds,
+        as this one does)."""
         dev = device or (_context if isinstance(_context, str) else None) or 'cuda:0'
         self.tracker = Tracker(self, backend=backend, device=dev, compile=compile,
                                waves_per_eu=waves_per_eu, arithmetic=arithmetic)

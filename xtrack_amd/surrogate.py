@@ -4,9 +4,12 @@ the reference).
 A small MLP (16 -> 256 -> 256 -> 256 -> 1, ReLU) predicts log(survival
 turn) of a particle from its initial normalised coordinates and features of
 its first turns (tracked by the plain tracker).  Its products run on the
-matrix cores through xtm_gemm_bf16 (BF16 operands, FP32 accumulation),
-forward and backward; the FP32 master weights, the bias and loss sums and
-the Adam update are torch tensor operations on the same device.
+matrix cores (BF16 operands, FP32 accumulation), forward and backward, with
+FP32 master weights.  The default network predicts in one kernel
+(xtm_mlp_forward); training steps of at most 8 layers are library calls
+(xtm_mlp_train_forward, xtm_mlp_train_backward, xtm_adam_step); any other
+network runs product by product (xtm_gemm_bf16) with its sums and updates
+as tensor operations on the same device.
 
 The screened scan (``screened_da_scan``, over many lattices at once on the
 batch tracker) tracks every grid particle for the feature turns with the
