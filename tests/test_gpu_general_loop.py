@@ -17,7 +17,9 @@ def test_lines_against_the_oracle(name):
     lc.build_tracker(backend=OracleBackend())
     p = random_particles(5003, seed=3, scale=1.5e-3, p0c=7e12)
     for kw in (dict(num_turns=3), dict(num_turns=2, ele_start=3, ele_stop=9),
-               dict(num_turns=2, turn_by_turn_monitor=True), dict(num_turns=2, backtrack=True)):
+               dict(num_turns=2, turn_by_turn_monitor=True),
+               dict(num_turns=1, turn_by_turn_monitor='ONE_TURN_EBE'),
+               dict(num_turns=2, backtrack=True)):
         pg, pc = p.copy(_context='cuda:0'), p.copy()
         lg.track(pg, **kw)
         lc.track(pc, **kw)

@@ -1157,6 +1157,10 @@ int xt_generate_line_source(const std::vector<int64_t> &entry, const std::vector
     return line_source(entry, prog, waves_per_eu, options, src, rec_of_elem, err, false);
 }
 
+bool xt_source_has_units(const std::string &src) {
+    return src.find("xt::track_particle_units") != std::string::npos;
+}
+
 int xt_generate_backtrack_source(const std::vector<int64_t> &entry,
                                  const std::vector<double> &prog, int32_t waves_per_eu,
                                  std::string &src, std::vector<int32_t> &rec_of_elem,

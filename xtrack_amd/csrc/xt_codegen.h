@@ -43,6 +43,9 @@ int xt_generate_backtrack_source(const std::vector<int64_t> &entry,
                                  std::string &src, std::vector<int32_t> &rec_of_elem,
                                  std::string &err);
 
+// Whether a generated source tracks with the loop over units.
+bool xt_source_has_units(const std::string &src);
+
 // Source of a translation unit that tracks a batch of lines in one launch:
 // literal functions for records that serve several elements, else one
 // function per distinct element structure (the record code with its

@@ -462,7 +462,8 @@ XT_HD_COLD bool track_unit_general(const Runner run, const typename Runner::Key 
    for num_turns turns (track_particle_loop of xt_ops.h with the units of the
    file comment).  BT: backtracking; the runner's elements are then the line's
    in reverse order with their backtracking programs, and ele_start counts in
-   that order.  All lanes of a wave walk the units together; a lane without a
+   that order.  Element-by-element records (flag_monitor 2) are the host
+   build's: the library takes them on the interpreter.  All lanes of a wave walk the units together; a lane without a
    particle, or whose particle is lost, takes part without effect (alive
    false), so that the loops are scalar. */
 template <bool BT, class Runner>
