@@ -50,3 +50,24 @@ def test_compiled_with_or_without_units(n_patterns, units):
 
 def test_beyond_the_limit():
     assert _generate(_quads(2100))[0] == _native.XTM_ERR_UNSUPPORTED
+
+
+def test_bends_of_many_variants_share_structures():
+    """32 ring variants with as many bend strengths as cell counts: the bends
+    get structure functions, however their units' guards divide them."""
+    from test_batch import _free, _host_batch
+    from xtrack_amd import lattices
+    lines = [lattices.collider_variant(k) for k in range(32)]
+    lib, handles, b = _host_batch(lines)
+    try:
+        n = ctypes.c_int64()
+        _native.check(lib.xtm_batch_generate_source(b, 0, None, 0, ctypes.byref(n), None))
+        buf = ctypes.create_string_buffer(n.value + 1)
+        _native.check(lib.xtm_batch_generate_source(b, 0, buf, n.value + 1, ctypes.byref(n),
+                                                    None))
+    finally:
+        _free(lib, handles, b)
+    src = buf.value.decode()
+    body = [f for f in src.split('XT_GEN_FN void rec_')[1:]]
+    literal_bends = [f for f in body if 'xt::op_yoshida4(p, 0x' in f.split('\n}\n')[0]]
+    assert not literal_bends

@@ -670,6 +670,14 @@ std::string both(const std::string &general, const std::string &unit) {
     return general + '\n' + unit;
 }
 
+// the words of a record that its text loads (rp[k])
+std::vector<int64_t> loaded_words(const std::string &text) {
+    std::vector<int64_t> out;
+    for (size_t q = text.find("rp["); q != std::string::npos; q = text.find("rp[", q + 3))
+        out.push_back(std::strtoll(text.c_str() + q + 3, nullptr, 10));
+    return out;
+}
+
 /* with_units: general and unit code of every function; else general code
    alone, for the element loop. */
 int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
@@ -695,49 +703,89 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     }
     const bool all_literal = !keyed_pc && nl == 1 && n_distinct <= kLiteralAll;
     cs.keyed_pc = !all_literal;
-    // literal code of every record (program addresses relative to the
-    // record unless every record of a single line is literal).  Records share
-    // a function when their general and their unit code are both the same:
-    // the general code of OP_YOSHIDA6_BEND reads its constants from the
-    // record, so bends of different lengths can agree in it, while the unit
-    // code holds every constant as a literal.
-    struct Literal {
-        std::string general, unit, structure;
-        int64_t uses = 0;
+    // Structures: the general and the unit code of a record with its constants
+    // as loads.  Records of one op sequence differ in the latter where a form
+    // depends on the ranges of their constants.
+    struct Structure {
+        std::string general, unit;
+        std::vector<int64_t> words;     // the program words that the texts load
         bool small = false;
         int weight = 0;
     };
-    std::map<std::string, Literal> lits;                   // by both texts
-    std::vector<std::map<int64_t, const std::string *>> lit_key(nl);
-    std::map<std::string, int64_t> lits_of_struct;         // distinct literal codes
+    std::vector<Structure> structs;
+    std::map<std::string, int32_t> struct_of;               // by both texts
+    // Literals: the records of one structure with the same constants.  A record
+    // is known by its structure and the words loaded there, so that literal
+    // text is written only for the records that get a function of their own;
+    // a line of literal records only knows them by their text, with program
+    // addresses that are not relative to the record.
+    struct Literal {
+        size_t line;
+        int64_t pc, uses;
+        int32_t structure;
+        std::string general, unit;
+    };
+    std::map<std::string, Literal> lits;
+    std::vector<std::map<int64_t, std::pair<int32_t, const std::string *>>> record(nl);
+    // distinct literals of a structure; heavy records of one general code count
+    // together, since their units are many copies of long code otherwise
+    std::map<std::string, int64_t> lits_of_struct;
+    auto counted = [&](const Structure &v) {
+        return v.small ? both(v.general, v.unit) : v.general;
+    };
     int64_t gain = 0;
+    auto cannot = [&](size_t l, int64_t pc) {
+        err = "cannot generate code for line " + std::to_string(l) + " at program offset " +
+              std::to_string(pc);
+        return XTM_ERR_ARG;
+    };
+    auto write = [&](Literal &v) {
+        Gen g(*progs[v.line], v.pc, false, !all_literal);
+        FastGen f(*progs[v.line], false);
+        const bool ok = g.record(v.pc);
+        v.unit = unit(f, v.pc);
+        v.general = std::move(g.out);
+        return ok;
+    };
     for (size_t l = 0; l < nl; l++)
         for (auto &pu : uses[l]) {
-            Gen g(*progs[l], pu.first, false, !all_literal);
             Gen gs(*progs[l], pu.first, true);
-            FastGen f(*progs[l], false), fs(*progs[l], true);
-            if (!g.record(pu.first) || !gs.record(pu.first)) {
-                err = "cannot generate code for line " + std::to_string(l) +
-                      " at program offset " + std::to_string(pu.first);
-                return XTM_ERR_ARG;
-            }
-            const std::string fast = unit(f, pu.first), fast_struct = unit(fs, pu.first);
-            auto ins = lits.emplace(both(g.out, fast), Literal());
-            Literal &v = ins.first->second;
-            if (ins.second) {
-                v.general = g.out;
+            FastGen fs(*progs[l], true);
+            if (!gs.record(pu.first)) return cannot(l, pu.first);
+            const std::string fast = unit(fs, pu.first);
+            const auto st = struct_of.emplace(both(gs.out, fast), (int32_t)structs.size());
+            if (st.second) {
+                structs.emplace_back();
+                Structure &v = structs.back();
+                v.small = !gs.heavy && gs.cost <= kSmallCost;
+                v.weight = fs.weight(v.small);
+                v.words = loaded_words(gs.out);
+                for (int64_t k : loaded_words(fast)) v.words.push_back(k);
+                std::sort(v.words.begin(), v.words.end());
+                v.words.erase(std::unique(v.words.begin(), v.words.end()), v.words.end());
+                v.general = gs.out;
                 v.unit = fast;
-                // a structure is its general and its unit code: records of
-                // one op sequence differ in the latter where a form depends
-                // on the ranges of their constants
-                v.structure = both(gs.out, fast_struct);
-                v.small = !g.heavy && g.cost <= kSmallCost;
-                v.weight = f.weight(v.small);
-                lits_of_struct[v.structure]++;
             }
-            v.uses += pu.second;
-            gain += v.weight * pu.second;
-            lit_key[l][pu.first] = &ins.first->first;
+            const Structure &sv = structs[st.first->second];
+            Literal lit{l, pu.first, 0, st.first->second, {}, {}};
+            std::string key;
+            if (all_literal) {
+                if (!write(lit)) return cannot(l, pu.first);
+                key = both(lit.general, lit.unit);
+            } else {
+                key.assign(reinterpret_cast<const char *>(&lit.structure), sizeof lit.structure);
+                for (int64_t k : sv.words) {
+                    if (pu.first + k < 0 || pu.first + k >= (int64_t)progs[l]->size())
+                        return cannot(l, pu.first);
+                    key.append(reinterpret_cast<const char *>(&(*progs[l])[pu.first + k]),
+                               sizeof(double));
+                }
+            }
+            auto ins = lits.emplace(std::move(key), std::move(lit));
+            if (ins.second) lits_of_struct[counted(sv)]++;
+            ins.first->second.uses += pu.second;
+            gain += (int64_t)sv.weight * pu.second;
+            record[l][pu.first] = {st.first->second, &ins.first->first};
         }
     // The loop over units suits a set whose elements gain more by their unit
     // code than those without one lose by their out-of-line calls; the other
@@ -751,50 +799,48 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
     // A structure that the set holds with many different constants (the
     // bends of ring variants with different cell counts) gets one structure
     // function rather than a literal copy per constant set.
-    std::vector<std::pair<int64_t, const std::string *>> ranked;
-    for (auto &kv : lits)
-        if (all_literal ||
-            (kv.second.uses >= 2 && lits_of_struct[kv.second.structure] <= kLiteralPerStruct))
-            ranked.emplace_back(kv.second.uses, &kv.first);
-    std::stable_sort(ranked.begin(), ranked.end(),
-                     [](const auto &x, const auto &y) { return x.first > y.first; });
+    std::vector<std::pair<Literal *, const std::string *>> ranked;
+    for (auto &kv : lits) {
+        Literal &v = kv.second;
+        if (!all_literal &&
+            (v.uses < 2 || lits_of_struct[counted(structs[v.structure])] > kLiteralPerStruct))
+            continue;
+        if (!all_literal && !write(v)) return cannot(v.line, v.pc);
+        ranked.emplace_back(&v, &kv.first);
+    }
+    std::stable_sort(ranked.begin(), ranked.end(), [](const auto &x, const auto &y) {
+        return x.first->uses != y.first->uses ? x.first->uses > y.first->uses
+               : x.first->general != y.first->general ? x.first->general < y.first->general
+                                                       : x.first->unit < y.first->unit;
+    });
     if ((int64_t)ranked.size() > kLiteralMax) ranked.resize(kLiteralMax);
-    std::map<std::string, int32_t> fn_of_lit;
+    std::map<const std::string *, int32_t> fn_of_lit;       // by the key in lits
     for (auto &r : ranked) {
-        const Literal &v = lits[*r.second];
-        fn_of_lit.emplace(*r.second, (int32_t)cs.body.size());
-        cs.body.push_back(v.general);
-        cs.fast.push_back(v.unit);
-        cs.small.push_back(v.small);
+        fn_of_lit.emplace(r.second, (int32_t)cs.body.size());
+        cs.body.push_back(r.first->general);
+        cs.fast.push_back(r.first->unit);
+        cs.small.push_back(structs[r.first->structure].small);
     }
     // the other records: structure functions, and the records of each
-    std::map<std::string, int32_t> fn_of_struct;
+    std::map<int32_t, int32_t> fn_of_struct;
     std::map<int32_t, std::vector<std::pair<size_t, int64_t>>> records_of;
     recs.assign(nl, {});
     for (size_t l = 0; l < nl; l++) {
         std::map<int64_t, int32_t> fn_of_pc;
-        for (auto &pu : uses[l]) {
-            auto it = fn_of_lit.find(*lit_key[l][pu.first]);
+        for (auto &pr : record[l]) {
+            auto it = fn_of_lit.find(pr.second.second);
             if (it != fn_of_lit.end()) {
-                fn_of_pc.emplace(pu.first, it->second);
+                fn_of_pc.emplace(pr.first, it->second);
                 continue;
             }
-            Gen g(*progs[l], pu.first, true);
-            FastGen f(*progs[l], true);
-            if (!g.record(pu.first)) {
-                err = "cannot generate code for line " + std::to_string(l) +
-                      " at program offset " + std::to_string(pu.first);
-                return XTM_ERR_ARG;
-            }
-            const std::string fast = unit(f, pu.first);
-            auto ins = fn_of_struct.emplace(both(g.out, fast), (int32_t)cs.body.size());
+            auto ins = fn_of_struct.emplace(pr.second.first, (int32_t)cs.body.size());
             if (ins.second) {
-                cs.body.push_back(g.out);
-                cs.fast.push_back(fast);
+                cs.body.push_back(structs[pr.second.first].general);
+                cs.fast.push_back(structs[pr.second.first].unit);
                 cs.small.push_back(0);
             }
-            fn_of_pc.emplace(pu.first, ins.first->second);
-            records_of[ins.first->second].emplace_back(l, pu.first);
+            fn_of_pc.emplace(pr.first, ins.first->second);
+            records_of[ins.first->second].emplace_back(l, pr.first);
         }
         if ((int64_t)cs.body.size() > XT_CODEGEN_MAX_RECORDS) {
             err = "the code needs more than " + std::to_string(XT_CODEGEN_MAX_RECORDS) +
@@ -813,9 +859,7 @@ int build_code_set(const std::vector<const std::vector<int64_t> *> &entries,
         const size_t l0 = kv.second[0].first;
         const int64_t pc0 = kv.second[0].second;
         std::vector<char> shared;
-        const std::string &text = cs.fast[kv.first];
-        for (size_t q = text.find("rp["); q != std::string::npos; q = text.find("rp[", q + 3)) {
-            const int64_t k = std::strtoll(text.c_str() + q + 3, nullptr, 10);
+        for (int64_t k : loaded_words(cs.fast[kv.first])) {
             if (k >= (int64_t)shared.size()) shared.resize(k + 1, 0);
             shared[k] = 1;
         }
